@@ -1,5 +1,5 @@
 // The MoE layer for a batch of rows (speculative verify, prefill): router GEMM, per-row top-k, slots sorted by
-// expert, and grouped expert GEMMs on the matrix cores that decode each expert's EXL3 tiles once per 128-row chunk
+// expert, and grouped expert GEMMs on the matrix cores that decode each expert's EXL3 tiles once per 32- to 128-row chunk
 // and feed them to v_mfma_f32_32x32x16_f16 (reference kernels/prefill/pf_moe.metal:26-338 and
 // kernels/fn_moe.metal:677-884, driven by prefill.mm:235-276).
 //
@@ -8,7 +8,7 @@
 //   bat_route    per row: top-k, ties to the lower index, weights exp(l - l_max) / sum (kernels/fn_moe.metal:76-131)
 //   bat_hist     slots per expert: LDS histograms of slices of the route, merged with global atomics
 //   bat_scan     one workgroup: per-expert offsets of the
-//                expert-sorted slot list (the shared expert's rows last) and the list of 128-row chunks (expert,
+//                expert-sorted slot list (the shared expert's rows last) and the list of chunks (expert,
 //                first row, rows) the GEMMs run over (kernels/prefill/pf_moe.metal:26-83)
 //   bat_place_prep  one wave per slot: its place in its expert's rows (row order inside an expert does not change
 //                any result: every row is computed independently) and that row of the A operand,
@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "exl3_device.h"
 #include "ring_schedule.h"
@@ -35,11 +36,14 @@
 
 namespace ijah {
 
+static int moe_gemm_rows(int R, int ne, int topk);
+static int moe_batch_chunks(int R, int ne, int topk, bool shared);
+
 namespace {
 
 
 constexpr int kChunkRows = 128;   // rows of one GEMM chunk (4 matrix-core row blocks of 32)
-constexpr int kRowBlocks = kChunkRows / 32;
+constexpr int64_t kRows32Below = 25, kRows64Below = 51;  // rows per expert that take 32- and 64-row chunks
 
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ void dma16(const void *src, void *lds_dst) {
@@ -83,6 +87,16 @@ __device__ __forceinline__ bool xcd_item(int nitems, int &item) {
   const int b = blockIdx.x, xcd = b & 7, idx = b >> 3, q = nitems >> 3, r = nitems & 7;
   if (idx >= q + (xcd < r ? 1 : 0)) return false;
   item = xcd * q + min(xcd, r) + idx;
+  return true;
+}
+// The same for per-chunk items (per column blocks of each of nch chunks; grid 8 ceil(max chunks / 8) per): XCD x takes
+// the chunks c = x mod 8 from the last, so that the shared expert's full chunks, last in the list, start first and
+// spread over the XCDs.
+__device__ __forceinline__ bool xcd_chunk(int nch, int per, int &ch, int &sub) {
+  const int b = blockIdx.x, c = (b & 7) + 8 * ((b >> 3) / per);
+  if (c >= nch) return false;
+  ch = nch - 1 - c;
+  sub = (b >> 3) % per;
   return true;
 }
 }  // namespace
@@ -771,7 +785,7 @@ __global__ __launch_bounds__(256) void bat_prep_rows(MoeArgs a, const uint32_t *
 }
 
 // ---------------------------------------------------------------------------------------------------- grouped GEMM
-// One workgroup (8 waves, two per SIMD) multiplies a chunk of up to 128 expert-sorted rows of A by one tile pair (32
+// One workgroup (8 waves, two per SIMD) multiplies a chunk of up to NR expert-sorted rows of A by one tile pair (32
 // columns) per wave of the expert's re-laid matrix (IT k tiles, IT even), two k tiles per step. There are NA A
 // operands (fp16, kp order, row stride lda halves, the second at A + ahalf): wave w multiplies operand aidx. Both
 // stream through LDS rings: A (shared; each wave requests 16 of its rows) kDA steps ahead, and each wave's own B
@@ -785,43 +799,30 @@ template <int K>
 constexpr int kDA = K >= 6 ? 1 : 2;
 template <int K>
 constexpr int kDB = K >= 6 ? 3 : 5;
-// NR: rows of a chunk, 128 (4 row blocks) or 32 (1 row block, for at most 32 rows: a quarter of the A ring, so that
-// three workgroups share a CU)
+// NR: rows of a chunk (32, 64 or 128)
 template <int K, int NA, int NR = kChunkRows>
 struct GemmIo {
   static constexpr uint32_t TB = 32u * K;                  // bytes of one 16x16 tile
   static constexpr uint32_t PB = 2 * 2 * TB;               // a wave's B bytes per step (a pair x 2 k tiles)
   static constexpr uint32_t AB = NA * NR * 64;             // A bytes per step (NA x NR rows x 32 halves)
-  static constexpr int DA = kDA<K>, DB = kDB<K>;
+  static constexpr int DA = NR == 64 ? 1 : kDA<K>, DB = NR == 64 ? 3 : kDB<K>;
   static constexpr int RA = DA + 1, RB = DB + 1;           // ring slots
   static constexpr uint32_t LDS_RING = RA * AB + kWavesG * RB * PB;
-  // the epilogues: row-major, 32 x 256 floats; transposed (NR = 128 only), 32 x 32 float tiles with a 36-float row
-  // pitch: 8 (down), 8 + 4 (gate/up)
-  static constexpr uint32_t EPI = NR == kChunkRows ? (NA == 2 ? 12u : 8u) * 32u * 36u * 4u : 32u * 256u * 4u;
+  // the epilogues: row-major, 32 x 256 floats; transposed, 8 tiles of 32 x 32 floats with a 36-float row pitch
+  static constexpr uint32_t EPI = 8u * 32u * 36u * 4u;
   static constexpr uint32_t LDS = LDS_RING > EPI ? LDS_RING : EPI;
-  // requests per A step: NR = 128, each wave loads 16 rows of each operand; NR = 32, each wave one slice of
-  // NA NR / 8 rows (its lanes past 4 rows each idle)
-  static constexpr int OA = NR == kChunkRows ? NA : 1, OB = (PB + 1023) / 1024;
+  static constexpr int RW = NA * NR / kWavesG;             // rows of A each wave requests per step
+  static constexpr int OA = (RW + 15) / 16, OB = (PB + 1023) / 1024;  // requests per step (16 rows of A each)
   static constexpr int NRB = NR / 32;
   static_assert(LDS <= 81920, "two workgroups per CU");
-  static_assert(NR == kChunkRows || (NR == 32 && LDS <= 53248), "three workgroups per CU at 32 rows");
+  static_assert(NR == kChunkRows || LDS <= 53248, "three workgroups per CU up to 64 rows");
   static_assert(RB % RA == 0 && DB > DA, "ring shapes");
 };
-template <int OA, int OB, int DA, int DB>
-__device__ __forceinline__ void wait_step(int t, int NS) {
-  static_assert(kAfterSteady<OA, OB, DA> <= 15, "vmcnt immediate");
-  if (steady_step<DB>(t, NS))
-    __builtin_amdgcn_s_waitcnt(0x0F70 | kAfterSteady<OA, OB, DA>);
-  else
-    wait_vm15(after_step<OA, OB, DA, DB>(t, NS));
-}
-
-// decodes the lane's B operand for both k tiles of one step straight from the ring bytes src
+// the trellis words of the lane's B operand for both k tiles of one step, from the ring bytes src
 template <int K>
-__device__ __forceinline__ void decode_step(const uint8_t *src, const BLane<K> &B, f16x8 (&bf)[2]) {
+__device__ __forceinline__ void read_step(const uint8_t *src, const BLane<K> &B, TileWords (&w)[4]) {
   constexpr int TW = 8 * K;
   const uint32_t *T = (const uint32_t *)src + B.tile * TW;
-  TileWords w[4];
 #pragma unroll
   for (int u = 0; u < 2; u++) {
     const uint32_t *Tu = T + u * 2 * TW;
@@ -832,13 +833,14 @@ __device__ __forceinline__ void decode_step(const uint8_t *src, const BLane<K> &
     w[2 * u + 1].w1 = Tu[B.g1.i1];
     w[2 * u + 1].w2 = kThreeWords<K> ? Tu[B.g1.i2] : 0u;
   }
-#pragma unroll
-  for (int u = 0; u < 2; u++) {
-    f16x2 l0, h0, l1, h1;
-    decode4<K>(w[2 * u], B.g0.sh, l0, h0);
-    decode4<K>(w[2 * u + 1], B.g1.sh, l1, h1);
-    bf[u] = f16x8{l0.x, l0.y, h0.x, h0.y, l1.x, l1.y, h1.x, h1.y};
-  }
+}
+// the B operand of k tile u of the step, decoded from its words
+template <int K>
+__device__ __forceinline__ f16x8 decode_half(const TileWords (&w)[4], int u, const BLane<K> &B) {
+  f16x2 l0, h0, l1, h1;
+  decode4<K>(w[2 * u], B.g0.sh, l0, h0);
+  decode4<K>(w[2 * u + 1], B.g1.sh, l1, h1);
+  return f16x8{l0.x, l0.y, h0.x, h0.y, l1.x, l1.y, h1.x, h1.y};
 }
 
 // quarter swizzle of A row r: distinct 16-byte bank groups for rows r .. r + 7 (eight lanes of a 128-byte read phase)
@@ -850,7 +852,7 @@ __device__ __forceinline__ int a_swz(int r) { return ((r >> 1) ^ ((r >> 3) & 1))
 // instead of one chain: each k chunk's sum a chain of 8 MFMAs from zero, the chunk sums folded left in groups of FG,
 // the group sums folded left (FG at least the chunk count: one left fold over the chunks).
 template <int K, int NA, bool TR = false, int NR = kChunkRows, int FG = 0>
-__device__ void chunk_gemm(const uint16_t *A, int lda, int ahalf, int aidx, int nrows, const uint8_t *tr, int IT,
+__device__ __forceinline__ void chunk_gemm(const uint16_t *A, int lda, int ahalf, int aidx, int nrows, const uint8_t *tr, int IT,
                            int pair, uint8_t *lds, f32x16 (&acc)[NR / 32], uint64_t *dbg, int kt0, int nkt) {
   using Io = GemmIo<K, NA, NR>;
   constexpr int NRB = Io::NRB;
@@ -867,25 +869,26 @@ __device__ void chunk_gemm(const uint16_t *A, int lda, int ahalf, int aidx, int 
     for (int i = 0; i < 16; i++) acc[rb][i] = 0.f;
   static_assert(FG == 0 || !TR, "the one-row order on row-major products");
   f32x16 grp[FG ? NRB : 1], tot[FG ? NRB : 1];  // FG: the open group's fold, the closed groups' fold
-  // A(t): NR = 128: 16 rows of this wave per operand; NR = 32: the wave's slice of RW = 4 NA rows of operand
-  // (RW w) / 32. Row r's 64 bytes (four 16-byte quarters q: k 8q .. 8q + 7) sit at r * 64 with quarter q in position
-  // q ^ a_swz(r), so that a read of one quarter of consecutive rows is free of bank conflicts. DMA lane l fills
-  // position l % 4 of row r0 + l / 4 (r0 the wave's first row). Stream addresses are a wave-uniform base plus a fixed
-  // per-lane offset.
-  constexpr int RW = NR == kChunkRows ? 16 : 4 * NA;
-  const int ao = NR == kChunkRows ? 0 : (wave * RW) / NR, r0 = NR == kChunkRows ? wave * 16 : (wave * RW) % NR;
-  const int rr = min(r0 + (lane >> 2), nrows - 1);
-  const uint32_t a_off = (uint32_t)(rr * lda + ((lane & 3) ^ a_swz(r0 + (lane >> 2))) * 8) * 2;
+  // A(t): the wave's RW rows of the NA x NR, 16 per request. Row r's 64 bytes (four 16-byte quarters q: k 8q .. 8q + 7)
+  // sit at r * 64 with quarter q in position q ^ a_swz(r), so that a read of one quarter of consecutive rows is free of
+  // bank conflicts. DMA lane l fills position l % 4 of row r0 + l / 4 (r0 the request's first row). Stream addresses
+  // are a wave-uniform base plus a fixed per-lane offset; for rows past the chunk it lies beyond the descriptor's
+  // range, so nothing is read for them (48 rows of a 32-row chunk GEMM: 230 -> 221 us a layer).
+  constexpr int RW = Io::RW;
+  const int ao = (wave * RW) / NR, r0 = (wave * RW) % NR;
+  uint32_t a_off[Io::OA];
+#pragma unroll
+  for (int o = 0; o < Io::OA; o++) {
+    const int rr = r0 + 16 * o + (lane >> 2);
+    a_off[o] = rr < nrows ? (uint32_t)(rr * lda + ((lane & 3) ^ a_swz(rr)) * 8) * 2 : 0xFFFFFFF0u;
+  }
   const __amdgpu_buffer_rsrc_t ra = stream_rsrc(A + kt0 * 16);
   auto issue_a = [&](int t, int slot) {
-    if constexpr (NR == kChunkRows) {
 #pragma unroll
-      for (int o = 0; o < NA; o++)
-        dma16_buf(ra, a_off, (uint32_t)(o * ahalf * 2 + t * 64), ring_a + slot * Io::AB + o * NR * 64 + wave * 1024);
-    } else {
-      if (lane < 4 * RW)  // one request per wave and step (the idle lanes load nothing)
-        dma16_buf(ra, a_off, (uint32_t)(ao * ahalf * 2 + t * 64), ring_a + slot * Io::AB + ao * NR * 64 + r0 * 64);
-    }
+    for (int o = 0; o < Io::OA; o++)
+      if (RW - 16 * o >= 16 || lane < 4 * (RW - 16 * o))  // (the last request's idle lanes load nothing)
+        dma16_buf(ra, a_off[o], (uint32_t)(ao * ahalf * 2 + t * 64),
+                  ring_a + slot * Io::AB + (ao * NR + r0 + 16 * o) * 64);
   };
   // B(t): the wave's pair at k tiles 2t, 2t + 1 (contiguous)
   const __amdgpu_buffer_rsrc_t rb =
@@ -898,60 +901,81 @@ __device__ void chunk_gemm(const uint16_t *A, int lda, int ahalf, int aidx, int 
   };
   // step s begins when A(s) and B(s) are in: every wave's rows of A(s) landed (barrier), and every wave has read
   // its fragments of A(s - 1), whose ring slot the step's A request then reuses. sb = s mod RB (compile-time).
-  f16x8 bf[2];
-  auto begin_step = [&](int s, int sb) {
-    wait_step<Io::OA, Io::OB, DA, Io::DB>(s, NS);
-    lds_barrier();
-    if (s + DA < NS) issue_a(s + DA, (sb + DA) % Io::RA);
-    if (s + Io::DB < NS) issue_b(s + Io::DB, (sb + Io::DB) % Io::RB);
-    decode_step<K>(ring_b + sb * Io::PB, BL, bf);
+  const uint8_t *a_lane = ring_a + aidx * NR * 64 + (lane & 31) * 64;
+  const int q0 = ((lane >> 5) ^ a_swz(lane & 31)) * 16, q1 = ((2 + (lane >> 5)) ^ a_swz(lane & 31)) * 16;
+  auto step = [&](auto nbc, int s, int sb) {
+    constexpr int NB = decltype(nbc)::value;  // the chunk's row blocks: no branch inside the step
+    TileWords w[4];
+    // (the steady count also serves the first DB steps, where more requests than that follow step s's data)
+    if (s + Io::DB < NS) {
+      __builtin_amdgcn_s_waitcnt(0x0F70 | kAfterSteady<Io::OA, Io::OB, DA>);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      read_step<K>(ring_b + sb * Io::PB, BL, w);
+      asm volatile("s_barrier" ::: "memory");
+      issue_a(s + DA, (sb + DA) % Io::RA);
+      issue_b(s + Io::DB, (sb + Io::DB) % Io::RB);
+    } else {
+      wait_vm15(after_step<Io::OA, Io::OB, DA, Io::DB>(s, NS));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      read_step<K>(ring_b + sb * Io::PB, BL, w);
+      asm volatile("s_barrier" ::: "memory");
+      if (s + DA < NS) issue_a(s + DA, (sb + DA) % Io::RA);
+    }
+    const uint8_t *at = a_lane + (sb % Io::RA) * Io::AB;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      f16x8 af[NB];
+#pragma unroll
+      for (int rb = 0; rb < NB; rb++) af[rb] = *(const f16x8 *)(at + rb * 2048 + (h ? q1 : q0));
+      const f16x8 bf = decode_half<K>(w, h, BL);
+#pragma unroll
+      for (int rb = 0; rb < NB; rb++)  // the row blocks of one k tile: no two dependent MFMAs adjacent
+        acc[rb] = TR ? __builtin_amdgcn_mfma_f32_32x32x16_f16(bf, af[rb], acc[rb], 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f32_32x32x16_f16(af[rb], bf, acc[rb], 0, 0, 0);
+    }
+    if constexpr (FG > 0) {
+      if (((s + 1) & 3) == 0) {  // k chunk (s + 1) / 4 - 1 complete (4 steps of 2 k tiles)
+        const int c = (s + 1) / 4 - 1, ci = c % FG;
+#pragma unroll
+        for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            grp[rb][i] = ci == 0 ? acc[rb][i] : grp[rb][i] + acc[rb][i];
+            acc[rb][i] = 0.f;
+          }
+        if (ci == FG - 1) {
+#pragma unroll
+          for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) tot[rb][i] = c + 1 == FG ? grp[rb][i] : tot[rb][i] + grp[rb][i];
+        }
+      }
+    }
   };
   for (int j = 0; j < Io::DB && j < NS; j++) {
     if (j < DA) issue_a(j, j % Io::RA);
     issue_b(j, j);
   }
-  begin_step(0, 0);
-  const uint8_t *a_lane = ring_a + aidx * NR * 64 + (lane & 31) * 64;
-  const int q0 = ((lane >> 5) ^ a_swz(lane & 31)) * 16, q1 = ((2 + (lane >> 5)) ^ a_swz(lane & 31)) * 16;
-  for (int t0 = 0; t0 < NS; t0 += U) {
+  auto loop = [&](auto nbc) {
+    for (int t0 = 0; t0 < NS; t0 += U) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int t = t0 + u;
-      if (t >= NS) break;
-      const uint8_t *at = a_lane + (u % Io::RA) * Io::AB;
-      const f16x8 b0 = bf[0], b1 = bf[1];
-#pragma unroll
-      for (int h = 0; h < 2; h++) {  // k tile h of the step for every row block: no two dependent MFMAs adjacent
-        f16x8 af[NRB];
-#pragma unroll
-        for (int rb = 0; rb < NRB; rb++) af[rb] = *(const f16x8 *)(at + rb * 2048 + (h ? q1 : q0));
-#pragma unroll
-        for (int rb = 0; rb < NRB; rb++)
-          if (rb < nrb)
-            acc[rb] = TR ? __builtin_amdgcn_mfma_f32_32x32x16_f16(h ? b1 : b0, af[rb], acc[rb], 0, 0, 0)
-                         : __builtin_amdgcn_mfma_f32_32x32x16_f16(af[rb], h ? b1 : b0, acc[rb], 0, 0, 0);
+      for (int u = 0; u < U; u++) {
+        if (t0 + u >= NS) break;
+        step(nbc, t0 + u, u);
       }
-      if constexpr (FG > 0) {
-        if (((t + 1) & 3) == 0) {  // k chunk (t + 1) / 4 - 1 complete (4 steps of 2 k tiles)
-          const int c = (t + 1) / 4 - 1, ci = c % FG;
-#pragma unroll
-          for (int rb = 0; rb < NRB; rb++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-              grp[rb][i] = ci == 0 ? acc[rb][i] : grp[rb][i] + acc[rb][i];
-              acc[rb][i] = 0.f;
-            }
-          if (ci == FG - 1) {
-#pragma unroll
-            for (int rb = 0; rb < NRB; rb++)
-#pragma unroll
-              for (int i = 0; i < 16; i++) tot[rb][i] = c + 1 == FG ? grp[rb][i] : tot[rb][i] + grp[rb][i];
-          }
-        }
-      }
-      // the matrix cores run while the next step's tiles decode
-      if (t + 1 < NS) begin_step(t + 1, (u + 1) % U);
     }
+  };
+  if constexpr (NRB == 1) {
+    loop(std::integral_constant<int, 1>{});
+  } else {
+    if (nrb == 1)
+      loop(std::integral_constant<int, 1>{});
+    else if (NRB == 2 || nrb == 2)
+      loop(std::integral_constant<int, 2>{});
+    else if (nrb == 3)
+      loop(std::integral_constant<int, NRB < 3 ? 1 : 3>{});
+    else
+      loop(std::integral_constant<int, NRB < 4 ? 1 : 4>{});
   }
   if constexpr (FG > 0) {
     const int nc = NS / 4;  // k chunks; closed groups, and an open one past them
@@ -1018,13 +1042,11 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
                                                      const uint32_t *rows, const uint16_t *xh, uint16_t *hh) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int nib = a.inter / 128;
-  int item;
-  if (!xcd_item((int)bk[3 * (a.ne + 1)] * nib, item)) return;
-  const int ch = item / nib, ib = item % nib;
+  int ch, ib;
+  if (!xcd_chunk((int)bk[3 * (a.ne + 1)], nib, ch, ib)) return;
   const int e = (int)chunks[3 * ch], row0 = (int)chunks[3 * ch + 1], nrows = (int)chunks[3 * ch + 2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, proj = wave >> 2;
   const uint8_t *blk = expert_block(a, e);
-  static_assert(!TR || NR == kChunkRows, "transposed products at 128-row chunks");
   constexpr int NRB = NR / 32;
   f32x16 acc[NRB];
   const uint16_t *A = xh + (uint64_t)row0 * 2 * a.hid;  // [row][gate | up][hid]
@@ -1097,8 +1119,8 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
   const uint16_t *pg = (const uint16_t *)(blk + sv_of(a, e, 0)) + c0, *pu = (const uint16_t *)(blk + sv_of(a, e, 1)) + c0;
   const uint16_t *pd = (const uint16_t *)(blk + su_of(a, e, 2)) + c0;
   const float sc = a.sc_inter;
-  // LDS: 8 step-1 tiles then 4 step-2 tiles of 32 rows x 32 elements, row pitch 36 floats
-  float *x1 = (float *)lds, *x2 = x1 + 8 * 32 * 36;
+  // LDS: 8 step-1 tiles of 32 rows x 32 elements, row pitch 36 floats; the 4 step-2 tiles take their place
+  float *x1 = (float *)lds, *x2 = x1;
   const int nrb = (nrows + 31) / 32;
 #pragma unroll
   for (int rb = 0; rb < NRB; rb++) {
@@ -1109,6 +1131,7 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
     for (int g = 0; g < 4; g++)
       *(float4 *)(x1 + (wave * 32 + n) * 36 + 8 * g + 4 * h) = make_float4(T[4 * g], T[4 * g + 1], T[4 * g + 2], T[4 * g + 3]);
     __syncthreads();
+    f32x16 T2;
     if (wave < 4) {
       f32x16 hv;
 #pragma unroll
@@ -1137,7 +1160,10 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
           hv[4 * g + r] = gg * __builtin_amdgcn_rcpf(1.f + __expf(-gg)) * uu * (float)sdv[r];
         }
       }
-      const f32x16 T2 = h32_tile(hv, hA2, lane);
+      T2 = h32_tile(hv, hA2, lane);
+    }
+    __syncthreads();  // the step-1 tiles are read
+    if (wave < 4) {
 #pragma unroll
       for (int g = 0; g < 4; g++)
         *(float4 *)(x2 + (q * 32 + n) * 36 + 16 * h + 4 * g) = make_float4(T2[4 * g], T2[4 * g + 1], T2[4 * g + 2], T2[4 * g + 3]);
@@ -1170,9 +1196,8 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
                                                    const uint32_t *rows, const uint16_t *hh, float *dnw) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int nob = a.hid / 256;
-  int item;
-  if (!xcd_item((int)bk[3 * (a.ne + 1)] * nob, item)) return;
-  const int ch = item / nob, ob2 = item % nob;
+  int ch, ob2;
+  if (!xcd_chunk((int)bk[3 * (a.ne + 1)], nob, ch, ob2)) return;
   const int e = (int)chunks[3 * ch], row0 = (int)chunks[3 * ch + 1], nrows = (int)chunks[3 * ch + 2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint8_t *blk = expert_block(a, e);
@@ -1181,7 +1206,6 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
   __shared__ float m_w[kChunkRows];
   const int mt = threadIdx.x;
   const uint32_t sl = mt < nrows ? rows[row0 + mt] : 0u;
-  static_assert(!TR || NR == kChunkRows, "transposed products at 128-row chunks");
   constexpr int NRB = NR / 32;
   f32x16 acc[NRB];
   const uint16_t *A = hh + (uint64_t)row0 * a.inter;
@@ -1560,26 +1584,28 @@ void launch_gemms_as(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
   // the routed (K) and shared (KS) chunks use ring layouts of their own widths: room for the larger of each
   const size_t lg = std::max(GemmIo<K, 2, NR>::LDS, GemmIo<KS, 2, NR>::LDS);
   const size_t ld = std::max(GemmIo<K, 1, NR>::LDS, GemmIo<KS, 1, NR>::LDS);
-  hipLaunchKernelGGL((bat_gateup<K, KS, TR, NR, EX>), dim3((b.max_chunks * (a.inter / 128) + 7) & ~7),
+  const int most = moe_batch_chunks(a.R, a.ne, a.topk, a.nslot > a.topk), g8 = (most + 7) / 8 * 8;
+  IJ_CHECK(most <= b.max_chunks, "grouped GEMM: %d chunks, room for %d", most, b.max_chunks);
+  hipLaunchKernelGGL((bat_gateup<K, KS, TR, NR, EX>), dim3(g8 * (a.inter / 128)),
                      dim3(64 * kWavesG), lg, s, a, b.bk, b.chunks, b.rows, b.xh, b.hh);
-  hipLaunchKernelGGL((bat_down<K, KS, TR, NR, EX>), dim3((b.max_chunks * (a.hid / 256) + 7) & ~7), dim3(64 * kWavesG),
+  hipLaunchKernelGGL((bat_down<K, KS, TR, NR, EX>), dim3(g8 * (a.hid / 256)), dim3(64 * kWavesG),
                      ld, s, a, b.bk, b.chunks, b.rows, b.hh, b.dnw);
 }
-// Chunks of many rows (8 or more per routed expert on average) take the transposed products and the matrix-core
-// Hadamard epilogues; chunks of a row or two (speculative verify) the row-major products and lane butterflies, which
-// cost less there.
-// At most 32 rows (speculative verify) no chunk exceeds 32 rows: the one-row-block form, three workgroups per CU,
-// with the one-row step's arithmetic (every row bit-identical to the row run alone).
+// Rows of a chunk (moe_gemm_rows) fix the form: 32-row chunks (eight waves per SIMD, row-major products and lane
+// butterflies, whose cost follows the rows) and, above, the transposed products and matrix-core Hadamard epilogues.
+// At most 32 rows (speculative verify) take the one-row step's arithmetic (every row bit-identical to the row run
+// alone).
 template <int K, int KS>
 void launch_gemms(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
+  const int rows = moe_gemm_rows(a.R, a.ne, a.topk);
   if (moe_batch_exact(a))
     launch_gemms_as<K, KS, false, 32, true>(a, b, s);
-  else if (a.R <= 32)
+  else if (a.R <= 32 || rows == 32)
     launch_gemms_as<K, KS, false, 32>(a, b, s);
-  else if ((int64_t)a.R * a.topk >= 8LL * a.ne)
-    launch_gemms_as<K, KS, true, kChunkRows>(a, b, s);
+  else if (rows == 64)
+    launch_gemms_as<K, KS, true, 64>(a, b, s);
   else
-    launch_gemms_as<K, KS, false, kChunkRows>(a, b, s);
+    launch_gemms_as<K, KS, true, kChunkRows>(a, b, s);
 }
 }  // namespace
 
@@ -1626,7 +1652,7 @@ static void gemm_attrs_all() {
   gemm_attrs<K, KS, true, kChunkRows>();
   gemm_attrs<K, KS, false, 32, true>();
   gemm_attrs<K, KS, false, 32>();
-  gemm_attrs<K, KS, false, kChunkRows>();
+  gemm_attrs<K, KS, true, 64>();
 }
 void init_batch_attrs() {
   IJ_HIP(hipFuncSetAttribute((const void *)&bat_place_prep, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPrepLds));
@@ -1660,8 +1686,28 @@ bool moe_batch_supported(int K, int KS, int hid, int inter, int ne, int topk) {
   const bool ks = (K >= 4 && K <= 6) && (KS >= 4 && KS <= 6);
   return ks && hid % 256 == 0 && inter % 128 == 0 && hid <= 8192 && inter <= 4096 && ne < 1024 && topk <= 32;
 }
+// Rows of a GEMM chunk by the routed rows per expert m. A chunk decodes its expert's weights once, whatever its rows,
+// so a chunk should hold an expert's rows whole; a smaller one runs with more workgroups per CU (4, 3 and 2) and
+// fetches fewer rows that are not there. Measured, hidden 2048 x inter 512, K5, us per layer at m = 4 / 14 / 20 / 25 /
+// 33 / 49: 32 rows 331 / 416 / 453 / 504 / 640 / 843, 64 rows 358 / 450 / 474 / 500 / 556 / 653, 128 rows 392 / 483 /
+// 505 / 530 / 586 / 677.
+static int moe_gemm_rows(int R, int ne, int topk) {
+  const int64_t m = (int64_t)R * topk / ne;
+  return m < kRows32Below ? 32 : m < kRows64Below ? 64 : kChunkRows;
+}
+// the chunks of R rows are at most one per touched expert, one per further whole chunk of rows, and the shared expert's
+static int moe_batch_chunks(int R, int ne, int topk, bool shared) {
+  const int rows = moe_gemm_rows(R, ne, topk);
+  return (int)std::min<int64_t>(ne, (int64_t)R * topk) + R * topk / rows + (shared ? (R + rows - 1) / rows : 0);
+}
+// the most that any row count up to R needs: each chunk size at the most rows that take it
 int moe_batch_max_chunks(int R, int ne, int topk, bool shared) {
-  return (R * topk + kChunkRows - 1) / kChunkRows + ne + (shared ? (R + kChunkRows - 1) / kChunkRows : 0) + 1;
+  int most = moe_batch_chunks(R, ne, topk, shared);
+  for (int64_t below : {kRows32Below, kRows64Below}) {
+    const int64_t r = (below * ne - 1) / topk;  // the largest r with r topk / ne below it
+    if (r >= 1 && r < R) most = std::max(most, moe_batch_chunks((int)r, ne, topk, shared));
+  }
+  return most;
 }
 
 void launch_moe_batch(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
@@ -1694,7 +1740,7 @@ void launch_moe_batch(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
     const int self_count = a.R * a.topk < 4096;  // few slots: counted inside bat_scan
     if (!self_count) hipLaunchKernelGGL(bat_hist, dim3(kHistGroups), dim3(256), 0, s, a, b.bk);
     hipLaunchKernelGGL(bat_scan, dim3(1), dim3(1024), 0, s, a, b.bk, b.chunks, b.max_chunks, self_count,
-                       (uint32_t)kChunkRows);
+                       (uint32_t)moe_gemm_rows(a.R, a.ne, a.topk));
   }
   IJ_CHECK(a.had_hid == 128, "batched MoE: hidden size %d needs a 128-wide Hadamard", a.hid);
   if (few) {

@@ -29,10 +29,11 @@ constexpr int after_step(int t, int NS) {
   }
   return total - last;
 }
-// Steps t with DB <= t and t + DB < NS (both streams still issuing) wait with one compile-time count: A(t) is the
-// later request, followed by B(t - DA + DB) and DA - 1 full steps.
+// Steps t with t + DB < NS (both streams still issuing) wait with one compile-time count: from step DB on A(t) is the
+// later request, followed by B(t - DA + DB) and DA - 1 full steps; the first DB steps have more requests behind
+// theirs, so the same count waits a little longer there.
 template <int DB>
-constexpr bool steady_step(int t, int NS) { return t >= DB && t + DB < NS; }
+constexpr bool steady_step(int t, int NS) { return t + DB < NS; }
 template <int OA, int OB, int DA>
 constexpr int kAfterSteady = OB + (DA - 1) * (OA + OB);
 static_assert(after_step<2, 1, 2, 5>(5, 1000) == kAfterSteady<2, 1, 2> &&

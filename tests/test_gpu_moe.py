@@ -204,6 +204,25 @@ def test_moe_batch_row_block_forms(eng, oracle, R):
     assert np.array_equal(m.run(x), y)
 
 
+@pytest.mark.parametrize("R,K,Ks", [(99, 5, 5), (100, 4, 6), (203, 6, 4), (204, 5, 6)])
+def test_moe_batch_chunk_sizes(eng, oracle, R, K, Ks):
+    """Both sides of the row counts where the GEMM's chunks change size (8 experts, top-2: 24 and 25, 50 and 51 routed
+    rows per expert take 32-, 64-, 64- and 128-row chunks), on a layer whose buffers an R = 260 run sized first; then
+    rows that all route alike, so that two experts take every row in whole chunks and a remainder: each row is then
+    the same sums in the same order, so all come out alike, and as the row came out among others."""
+    print(f"moe batch chunk sizes R{R} K{K}/{Ks}", flush=True)
+    w = synth.moe_layer(900 + R, hid=512, inter=128, ne=8, topk=2, K=K, shared=True, Ks=Ks, sgate=True)
+    W = oracle.MoeWeights(w)
+    m = eng.moe_create(w)
+    rng = np.random.default_rng(901)
+    m.run(synth.bf16_values(rng, 260, 512))
+    x = synth.bf16_values(rng, R, 512)
+    y, _ = check_layer(eng, oracle, m, W, x, exact=False)
+    assert np.array_equal(m.run(x), y)
+    same = m.run(np.repeat(x[:1], R, 0))
+    assert np.array_equal(same, np.repeat(y[:1], R, 0))
+
+
 def test_moe_batch_matches_staged(eng, oracle):
     """The grouped path and the staged kernels compute the same layer for several rows."""
     w = synth.moe_layer(81, hid=2048, inter=512, ne=64, topk=10, K=5, shared=True, Ks=5, sgate=False)
