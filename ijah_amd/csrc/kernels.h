@@ -91,6 +91,7 @@ __host__ __device__ inline uint64_t q8_block_bytes(int hid, int inter) {
 // the 8-bit shared expert's two launches for the staged and batched paths (moe_q8.hip): q8gu, then q8o
 void launch_moe_q8(const MoeArgs &a, hipStream_t s);
 void launch_q8_bf16(const uint8_t *q8, uint16_t *bf, int hid, int inter, hipStream_t s);  // weight bytes -> bf16
+void init_q8_attrs();
 bool moe_q8_supported(int hid, int inter);
 void launch_moe_router(const MoeArgs &a, hipStream_t s);
 void launch_moe_gateup(const MoeArgs &a, hipStream_t s);

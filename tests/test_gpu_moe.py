@@ -559,3 +559,34 @@ def test_moe_fused_reference_shape(eng, oracle, shared, K, Ks):
         assert np.array_equal(m.run(x), y)
     if shared is True:  # the verify rows of this shape agree with the fused step, bit for bit
         _rows_match_one_row(m, synth.bf16_values(np.random.default_rng(202), 4, 2560), 4)
+
+
+def _rr(v):
+    return synth.bf16(v.astype(np.float32)).astype(np.uint32).__lshift__(16).view(np.float32).astype(np.float64)
+
+
+@pytest.mark.parametrize("hid,inter,R,whole", [(512, 128, 33, True), (512, 128, 65, False), (512, 256, 129, False),
+                                               (512, 1024, 2048, True), (512, 1024, 2049, False)])
+def test_moe_q8_many_rows_tiles(eng, hid, inter, R, whole):
+    """The 8-bit shared expert's matrix-core form against the dequantised matrices in f64: 64- and 128-row tiles (the
+    gate / up product of 2048 rows is the smallest that takes the larger), row remainders, and inputs that are bf16
+    values (whole: their split's low parts are zero and their products left out) or not. The outputs are bf16: sums that
+    differ in f32 (or, for inputs that are no bf16 values, by the split's 2^-17) round alike but for the few that lie at
+    a rounding boundary, so the distance stays well below one rounding's 2^-9."""
+    print(f"moe q8 tiles {hid}x{inter} R{R} whole={whole}", flush=True)
+    w = synth.moe_layer(950 + R, hid=hid, inter=inter, ne=4, topk=2, K=5, shared="q8", sgate=False)
+    m = eng.moe_create(w)
+    rng = np.random.default_rng(951)
+    x = synth.bf16_values(rng, R, hid) if whole else rng.standard_normal((R, hid)).astype(np.float32)
+    x[:, :128] = synth.bf16_values(rng, R, 128)  # one group without low parts among the others
+    m.run(x)
+
+    def lin(name, v, rows, inp):
+        q = np.ascontiguousarray(w[f"sq8_{name}.weight"]).view(np.uint8).reshape(rows, inp // 128, 128).astype(np.float64)
+        f = lambda a: (a.astype(np.uint32) << 16).view(np.float32).astype(np.float64)[..., None]  # noqa: E731
+        W = q * f(w[f"sq8_{name}.scales"]) + f(w[f"sq8_{name}.biases"])
+        return _rr(v @ W.reshape(rows, inp).T)
+
+    g, u = lin("gate", x.astype(np.float64), inter, hid), lin("up", x.astype(np.float64), inter, hid)
+    want = lin("down", _rr(g / (1 + np.exp(-g)) * u), hid, inter)
+    assert rel(m.read("shared_q8", R), want) < 1e-3
