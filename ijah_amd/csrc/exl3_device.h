@@ -195,18 +195,23 @@ __device__ __forceinline__ BLane<K> b_lane(uint32_t lane) {
 __device__ __forceinline__ uint32_t mcg_bits(uint32_t cw) {
   return ((cw * 0xCBAC1FEDu) & 0x8FFF8FFFu) ^ 0x3B603B60u;
 }
-// two codewords -> their fp16 values packed (c0 low, c1 high): each v_add_f16 (SDWA) adds the two halves of one r
-// and writes one half of the result, so no pack instruction is needed.
-__device__ __forceinline__ f16x2 mcg_pair(uint32_t c0, uint32_t c1) {
-  const uint32_t r0 = mcg_bits(c0), r1 = mcg_bits(c1);
-  uint32_t d;
-  asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
-      : "=v"(d)
-      : "v"(r0));
-  asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
-      : "+v"(d)
-      : "v"(r1));
-  return __builtin_bit_cast(f16x2, d);
+// four codewords -> their fp16 values packed (c0, c1 in a, c2, c3 in b, low halves first): each v_add_f16 (SDWA) adds
+// the two halves of one r and writes one half of the result, so no pack instruction is needed. One block, because a
+// half-register write has to be a VALU issue slot (or s_nop) ahead of its reader: here the writes alternate and an s_nop
+// ends the block. The compiler's own spacing after such a write counts a scalar instruction as the slot, and with only
+// an s_mov between the last write and v_mfma the matrix core read the old half (K 3 at 16 rows, one weight in 128).
+__device__ __forceinline__ void mcg_group(const uint32_t (&c)[4], f16x2 &a, f16x2 &b) {
+  const uint32_t r0 = mcg_bits(c[0]), r1 = mcg_bits(c[1]), r2 = mcg_bits(c[2]), r3 = mcg_bits(c[3]);
+  uint32_t d0, d1;
+  asm("v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+      "v_add_f16_sdwa %1, %4, %4 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+      "v_add_f16_sdwa %0, %3, %3 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+      "v_add_f16_sdwa %1, %5, %5 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+      "s_nop 0"
+      : "=&v"(d0), "=&v"(d1)
+      : "v"(r0), "v"(r1), "v"(r2), "v"(r3));
+  a = __builtin_bit_cast(f16x2, d0);
+  b = __builtin_bit_cast(f16x2, d1);
 }
 
 // The group's four codewords (15 bits each, at window bits K i .. K i + 14) from its words and shift.
@@ -236,8 +241,7 @@ template <int K>
 __device__ __forceinline__ void decode4(const TileWords &w, uint32_t sh, f16x2 &a, f16x2 &b) {
   uint32_t c[4];
   codewords4<K>(w, sh, c);
-  a = mcg_pair(c[0], c[1]);
-  b = mcg_pair(c[2], c[3]);
+  mcg_group(c, a, b);
 }
 
 // s_waitcnt vmcnt(n) for a run-time n (6-bit count: low 4 bits at [3:0], high 2 at [15:14]; n above 63 waits as for

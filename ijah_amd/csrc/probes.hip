@@ -154,7 +154,9 @@ __global__ __launch_bounds__(1024) void probe_lut(const uint8_t *tiles, int iter
   constexpr uint32_t B = kProbeTiles * 64 * K;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (uint32_t c = threadIdx.x; c < 32768u; c += blockDim.x) {
-    const f16x2 v = mcg_pair(c, c);
+    const uint32_t c4[4] = {c, c, c, c};
+    f16x2 v, v2;
+    mcg_group(c4, v, v2);
     lut[c] = v.x;
   }
   uint8_t *slot = lds + 65536 + wave * B;
