@@ -314,6 +314,27 @@ __device__ __forceinline__ f32x16 mfma_chunk(const uint8_t *tl, const _Float16 *
                                                    0);
   return acc;
 }
+// The same with the rows held for 8 or more distinct ones: row r's element i sits at r * 128 + (i ^ row_swz(r)), so that
+// the 16-byte reads of 8 consecutive rows fall in distinct banks (rows 256 bytes apart share theirs: an 8-way conflict
+// per read). xs: the chunk's rows, 128 halves each.
+__device__ __forceinline__ uint32_t row_swz(uint32_t r) { return (r & 7u) << 4; }
+template <int K, int NT>
+__device__ __forceinline__ f32x16 mfma_chunk_rows(const uint8_t *tl, const _Float16 *xs, int row, int nkt, f32x16 acc) {
+  const uint32_t x0 = (uint32_t)row * 128u + 8u * ((threadIdx.x & 63u) >> 5) + row_swz((uint32_t)row);
+  if (nkt == NT) {
+#pragma unroll
+    for (int kt = 0; kt < NT; kt++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const f16x8 *)(xs + (x0 ^ (16u * kt))), decode_pair<K>(tl, kt), acc,
+                                                   0, 0, 0);
+    return acc;
+  }
+#pragma unroll
+  for (int kt = 0; kt < NT; kt++)
+    if (kt < nkt)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const f16x8 *)(xs + (x0 ^ (16u * kt))), decode_pair<K>(tl, kt), acc,
+                                                   0, 0, 0);
+  return acc;
+}
 __device__ __forceinline__ float dot4(f16x2 a, f16x2 b, f16x4 x, float acc) {
   acc = __builtin_amdgcn_fdot2(a, f16x2{x.x, x.y}, acc, false);
   return __builtin_amdgcn_fdot2(b, f16x2{x.z, x.w}, acc, false);

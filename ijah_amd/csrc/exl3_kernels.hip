@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "exl3_device.h"
 #include "kernels.h"
@@ -612,10 +613,16 @@ __global__ __launch_bounds__(64) void lin_prep(LinArgs a) {
 // epilogue (reference kernels/trunk6/trunk6.metal:199-214, t6_finish). coherent: the partials were stored by other
 // workgroups of this launch (device-coherent loads); else by an earlier launch.
 // Rows r0, r0 + rs, .. (NR of them, those below R) of output block cb: each row's k-group partials folded left in
-// group order, H_out, svh and the epilogue. The partials of all NR rows are requested together (rounds of 8 groups
-// for one row, 4 for several), so a wave finishing several rows pays one round trip per round, not one per row.
-template <int NR>
-__device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool coherent) {
+// group order, H_out, svh and the epilogue. The partials of all NR rows are requested together, up to BMAX groups at a
+// time, so a wave finishing several rows pays one round trip per round, not one per row. sv: the lane's svh of the block
+// (lin_svh).
+__device__ __forceinline__ void lin_svh(const LinArgs &a, int cb, uint16_t (&sv)[2]) {
+  const int i0 = cb * 128 + (threadIdx.x & 63), i1 = i0 + 64;
+  sv[0] = a.svh[i0 < a.out ? i0 : 0];
+  sv[1] = a.svh[i1 < a.out ? i1 : 0];
+}
+template <int NR, int BMAX>
+__device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool coherent, const uint16_t (&sv)[2]) {
   const int lane = threadIdx.x & 63, OTp = a.OT + (a.OT & 1);
   const int i0 = cb * 128 + lane, i1 = i0 + 64;
   const bool m0 = i0 < a.out, m1 = i1 < a.out;
@@ -623,8 +630,8 @@ __device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool c
   float v0[NR], v1[NR];
 #pragma unroll
   for (int q = 0; q < NR; q++) v0[q] = v1[q] = 0.f;
-  constexpr int B = NR == 1 ? 8 : 4;  // groups requested together (2 NR B values in flight per lane)
-  for (int g0 = 0; g0 < a.S; g0 += B) {
+  auto fold = [&](auto bc, int g0) {  // groups g0 .. g0 + B - 1 (those below S)
+    constexpr int B = decltype(bc)::value;
     float t0[NR][B], t1[NR][B];
 #pragma unroll
     for (int q = 0; q < NR; q++) {
@@ -644,26 +651,35 @@ __device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool c
           v0[q] = g0 + j == 0 ? t0[q][j] : v0[q] + t0[q][j];
           v1[q] = g0 + j == 0 ? t1[q][j] : v1[q] + t1[q][j];
         }
-  }
+  };
+  constexpr int kFew = NR == 1 ? 8 : 4;
+  if (a.S <= kFew)
+    fold(std::integral_constant<int, kFew>{}, 0);
+  else
+    for (int g0 = 0; g0 < a.S; g0 += BMAX) fold(std::integral_constant<int, BMAX>{}, g0);
 #pragma unroll
   for (int q = 0; q < NR; q++) {
     const int r = r0 + q * rs;
     if (r >= a.R) break;
     float w0 = m0 ? v0[q] : 0.f, w1 = m1 ? v1[q] : 0.f;
     fwht2(w0, w1, lane, a.had_out, a.sc_out);
-    if (m0) lin_store(a, r, i0, w0 * h2f(a.svh[i0]));
-    if (m1) lin_store(a, r, i1, w1 * h2f(a.svh[i1]));
+    if (m0) lin_store(a, r, i0, w0 * h2f(sv[0]));
+    if (m1) lin_store(a, r, i1, w1 * h2f(sv[1]));
   }
 }
 __device__ void lin_finish_row(const LinArgs &a, int r, int cb, bool coherent) {
-  lin_finish_rows<1>(a, r, 1, cb, coherent);
+  uint16_t sv[2];
+  lin_svh(a, cb, sv);
+  lin_finish_rows<1, 8>(a, r, 1, cb, coherent, sv);
 }
-// the block's rows over the workgroup's 4 waves (wave c: rows c, c + 4, ..), four rows per request round
-__device__ void lin_finish_block(const LinArgs &a, int c, int cb) {
+// the block's rows over the workgroup's 4 waves (wave c: rows c, c + 4, ..), four rows per request round; B1 and B4: the
+// groups per round for one row and for four
+template <int B1, int B4>
+__device__ void lin_finish_block(const LinArgs &a, int c, int cb, const uint16_t (&sv)[2]) {
   if (a.R <= 4) {
-    if (c < a.R) lin_finish_rows<1>(a, c, 4, cb, true);
+    if (c < a.R) lin_finish_rows<1, B1>(a, c, 4, cb, true, sv);
   } else {
-    for (int r = c; r < a.R; r += 16) lin_finish_rows<4>(a, r, 4, cb, true);
+    for (int r = c; r < a.R; r += 16) lin_finish_rows<4, B4>(a, r, 4, cb, true, sv);
   }
 }
 
@@ -711,6 +727,13 @@ __global__ __launch_bounds__(256) void lin_mx(LinMulti m) {
   float *csum = (float *)(lds + 4 * lin_wave_lds<K, RT>());  // [4 chunks][RT rows][32 columns]
   const int e0 = kt0 * 16, i0 = e0 + lane, i1 = i0 + 64;    // the chunk's elements of this lane
   const int cb = p / 4;
+  // The finisher's svh is requested with the first loads, so that its latency is not paid after the hand-off, and the
+  // partials of up to 24 k groups (the reference's trunk has 20) in one round: up to 16 rows these small launches are
+  // chains of round trips (q, k, v and o of eight layers at one row 143 -> 133 us, the HC read of eight 153 -> 146). At 32
+  // rows, and in the kernels with many workgroups per output block, the registers cost more than the round trips
+  // (170 -> 178 us; vocabulary head at one row 82 -> 87): there svh is loaded late and the rounds are shorter.
+  uint16_t sv[2];
+  if constexpr (RT < 32) lin_svh(a, cb, sv);
   // 1. input rows and tiles
   float xv0[RT], xv1[RT], s0 = 0.f, s1 = 0.f;
   if (!a.xh_in && nkt > 0) {
@@ -762,7 +785,7 @@ __global__ __launch_bounds__(256) void lin_mx(LinMulti m) {
                                          (__attribute__((address_space(3))) void *)(tl + o), 16, 0, 0);
     if (a.xh_in) {  // rows r .. r + 3 per request: 16 lanes of 16 bytes each (the chunk's nkt * 32 bytes)
       for (int r = 0; r < R; r += 4) {
-        const int rr = r + (lane >> 4), q = lane & 15;
+        const int rr = r + (lane >> 4), q = (lane & 15) ^ (RT >= 8 ? (int)(row_swz(rr) >> 3) : 0);
         if (rr < R && q * 16 < nkt * 32)
           __builtin_amdgcn_global_load_lds((const void *)(a.xh + (uint64_t)rr * a.in + e0 + q * 8),
                                            (__attribute__((address_space(3))) void *)(xs + r * 128), 16, 0, 0);
@@ -812,14 +835,18 @@ __global__ __launch_bounds__(256) void lin_mx(LinMulti m) {
         if (r < R) {
           float v0 = xv0[r] * s0, v1 = xv1[r] * s1;
           fwht2(v0, v1, lane, a.had_in, a.sc_in);
-          xs[r * 128 + kp((uint32_t)lane)] = to_f16(v0);
-          xs[r * 128 + kp((uint32_t)lane + 64)] = to_f16(v1);
+          const uint32_t sw = RT >= 8 ? row_swz(r) : 0u;
+          xs[r * 128 + (kp((uint32_t)lane) ^ sw)] = to_f16(v0);
+          xs[r * 128 + (kp((uint32_t)lane + 64) ^ sw)] = to_f16(v1);
         }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the tiles (and rows) are in LDS
     // 2. the chunk's chain on the matrix cores
-    const _Float16 *xa = xs + min(lane & 31, R - 1) * 128 + 8 * (lane >> 5);
-    acc = mfma_chunk<K, kLinChunkKt>(tl, xa, nkt, acc);
+    const int row = min(lane & 31, R - 1);
+    if constexpr (RT >= 8)
+      acc = mfma_chunk_rows<K, kLinChunkKt>(tl, xs, row, nkt, acc);
+    else
+      acc = mfma_chunk<K, kLinChunkKt>(tl, xs + row * 128 + 8 * (lane >> 5), nkt, acc);
   }
   // 3. chunk sums (lane (n, h), value i: row 8 (i / 4) + 4 h + i % 4, column n) -> LDS; the group's fold -> partials
 #pragma unroll
@@ -841,7 +868,8 @@ __global__ __launch_bounds__(256) void lin_mx(LinMulti m) {
   uint32_t *ctr = a.cnt + (uint64_t)cb * kSyncStride;
   if (block_signal(ctr, &flag) != (uint32_t)(npb * a.S - 1)) return;
   if (threadIdx.x == 0) st_cg(ctr, 0u);
-  lin_finish_block(a, c, cb);
+  if constexpr (RT >= 32) lin_svh(a, cb, sv);
+  lin_finish_block<(RT <= 4 ? 24 : 8), (RT < 32 ? 8 : 4)>(a, c, cb, sv);
   if (a.epi.kind == 8)
     hc_fin_block(a, a.epi.ctr + (uint64_t)(cb % (a.epi.hid / 128)) * kSyncStride, a.epi.row0, a.epi.row0 + R, cb,
                  &flag);
@@ -926,7 +954,9 @@ __global__ __launch_bounds__(256) void lin_mxl(LinMulti m) {
   uint32_t *ctr = a.cnt + (uint64_t)cb * kSyncStride;
   if (block_signal(ctr, &flag) != (uint32_t)(npb - 1)) return;
   if (threadIdx.x == 0) st_cg(ctr, 0u);
-  lin_finish_block(a, c, cb);
+  uint16_t sv[2];
+  lin_svh(a, cb, sv);
+  lin_finish_block<8, 4>(a, c, cb, sv);
   if (a.epi.kind == 8)
     hc_fin_block(a, a.epi.ctr + (uint64_t)(cb % (a.epi.hid / 128)) * kSyncStride, a.epi.row0, a.epi.row0 + R, cb,
                  &flag);
@@ -966,7 +996,7 @@ __global__ __launch_bounds__(64 * NW) void lin_mxw(LinMulti m) {
                                            (__attribute__((address_space(3))) void *)(tl + o), 16, 0, 0);
     }
     for (int j = w; 4 * j < R; j += NW, n++) {
-      const int rr = 4 * j + (lane >> 4), q = lane & 15;
+      const int rr = 4 * j + (lane >> 4), q = (lane & 15) ^ (int)(row_swz(rr) >> 3);
       if (rr < R && q * 16 < nkt * 32)
         __builtin_amdgcn_global_load_lds((const void *)(a.xh + (uint64_t)rr * a.in + kt0 * 16 + q * 8),
                                          (__attribute__((address_space(3))) void *)(sb + 4 * j * 256), 16, 0, 0);
@@ -988,11 +1018,11 @@ __global__ __launch_bounds__(64 * NW) void lin_mxw(LinMulti m) {
     if (live) {
       const int kt0 = g * kLinGroupKt + c * kLinChunkKt, nkt = min(kLinChunkKt, IT - kt0);
       const uint8_t *sb = lds + (c & 1) * lin_mxw_stage<K, RT, NW>();
-      const _Float16 *xa = (const _Float16 *)sb + min(lane & 31, R - 1) * 128 + 8 * (lane >> 5);
       f32x16 acc;
 #pragma unroll
       for (int i = 0; i < 16; i++) acc[i] = 0.f;
-      acc = mfma_chunk<K, kLinChunkKt>(sb + RT * 256 + w * kLinChunkKt * 64 * K, xa, nkt, acc);
+      acc = mfma_chunk_rows<K, kLinChunkKt>(sb + RT * 256 + w * kLinChunkKt * 64 * K, (const _Float16 *)sb,
+                                            min(lane & 31, R - 1), nkt, acc);
 #pragma unroll
       for (int i = 0; i < 16; i++) v[i] = c == 0 ? acc[i] : v[i] + acc[i];
     }
@@ -1016,7 +1046,11 @@ __global__ __launch_bounds__(64 * NW) void lin_mxw(LinMulti m) {
     }
   }
   const int b = w >> 2;
-  if (last & (1u << b)) lin_finish_block(a, w & 3, (NW / 4) * bp + b);
+  if (last & (1u << b)) {
+    uint16_t sv[2];
+    lin_svh(a, (NW / 4) * bp + b, sv);
+    lin_finish_block<8, 4>(a, w & 3, (NW / 4) * bp + b, sv);
+  }
 }
 
 // lin_finish: the finisher of the staged path, grid R x ceil(out/128) (one workgroup per row and output block)
