@@ -102,161 +102,182 @@ __device__ __forceinline__ bool xcd_chunk(int nch, int per, int &ch, int &sub) {
 }  // namespace
 
 // ---------------------------------------------------------------------------------------------------- router
-// logits[r][c] = bf16(x[r] . router[c]) for c < ne + has_sgate on the matrix cores. A workgroup covers 32 rows and
-// CT 32-column tiles; its 8 waves are CT column tiles x KSP k splits, summed in LDS in split order. Few rows take
-// CT = 1, KSP = 8 (the k split keeps the chip busy); many rows take CT = 4, KSP = 2, so that each row of x is read
-// by a quarter as many workgroups. k steps of 16: x is split into bf16 hi + lo (x - hi rounded again), two MFMAs per
-// step, so the product carries about 16 mantissa bits of x: within f32 rounding of the reference's f32 dot for
-// these logits.
+// logits[r][c] = bf16(x[r] . router[c]) for c < ne + has_sgate on the matrix cores. k steps of 16: x is split into
+// bf16 hi + lo (x - hi rounded again), two MFMAs per step, so the product carries about 16 mantissa bits of x: within
+// f32 rounding of the reference's f32 dot for these logits.
+// Up to 511 rows a workgroup covers 32 rows x 32 columns; its 8 waves are 8 k splits (which keep the chip busy), summed
+// in LDS in split order.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-constexpr int kRouterWaves = 8;
-template <int CT>
-__global__ __launch_bounds__(512) void bat_router(MoeArgs a) {
-  constexpr int KSP = kRouterWaves / CT;
-  __shared__ float red[kRouterWaves][16][64];
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// A wave stages its own k range in LDS, 32 of k at a time (rows split on the way, whole 128-byte runs per load, kRsAhead
+// chunks' loads in flight): fragments loaded straight into registers, 16 scattered bytes a lane, kept the address units
+// busy for most of the 16.4 us that 48 rows took (now 13.3).
+constexpr int kRouterWaves = 8;  // k splits
+constexpr int kRsKc = 32, kRsPitch = kRsKc + 8, kRsAhead = 4;
+constexpr int kRsWave = 3 * 32 * kRsPitch * 2;  // LDS bytes per wave: hi, lo, columns
+__global__ __launch_bounds__(64 * kRouterWaves) void bat_router(MoeArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kRouterWaves * kRsWave];
+  float(*red)[16][64] = (float(*)[16][64])lds;
+  static_assert(sizeof(float) * 16 * 64 <= kRsWave, "the partial sums fit in the stages");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ncol = a.ne + a.has_sgate;
-  const int rt = blockIdx.x, ct = blockIdx.y * CT + wave % CT, ks = wave / CT;  // 32-row tile, 32-column tile
-  const bool live = ct * 32 < ncol;
+  const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;  // 32-row tile, 32-column tile
   const int m = lane & 31, h = lane >> 5;
-  const int row = min(rt * 32 + m, a.R - 1), col = min(ct * 32 + m, ncol - 1);
-  const int kn = a.hid / KSP, kb = ks * kn;  // this wave's k range (a multiple of 32 long)
-  static_assert(kRouterWaves % CT == 0, "waves per tile");
-  const float *xp = a.x + (uint64_t)row * a.hid + kb + 8 * h;
-  const uint16_t *wp = a.router + (uint64_t)col * a.hid + kb + 8 * h;
+  const int kn = a.hid / kRouterWaves, kb = wave * kn, nch = kn / kRsKc;  // this wave's k range (kn a multiple of 32)
+  __bf16 *xh = (__bf16 *)(lds + wave * kRsWave), *xl = xh + 32 * kRsPitch, *wl = xl + 32 * kRsPitch;
+  // lane: inputs 4 (lane % 8) .. + 3 of rows lane / 8 + 8 i, and 8 (lane % 4) .. + 7 of columns lane / 4 + 16 i
+  f32x4 xr[kRsAhead][4];
+  u32x4 wr[kRsAhead][2];
+  auto load = [&](int d, int c) {
+    const int k = kb + c * kRsKc;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      xr[d][i] = *(const f32x4 *)(a.x + (uint64_t)min(r0 + (lane >> 3) + 8 * i, a.R - 1) * a.hid + k + 4 * (lane & 7));
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      wr[d][i] = *(const u32x4 *)(a.router + (uint64_t)min(c0 + (lane >> 2) + 16 * i, ncol - 1) * a.hid + k +
+                                  8 * (lane & 3));
+  };
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; i++) acc[i] = 0.f;
-  // k steps in batches of U, the next batch's loads in flight while this one multiplies (kn is a multiple of 32,
-  // so batches are whole: kn / 16 steps, U = 2)
-  constexpr int U = 2;
-  float4 xv[2][U][2];
-  uint4 wv[2][U];
-  auto load = [&](int b, int k0) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      xv[b][u][0] = *(const float4 *)(xp + k0 + 16 * u);
-      xv[b][u][1] = *(const float4 *)(xp + k0 + 16 * u + 4);
-      wv[b][u] = *(const uint4 *)(wp + k0 + 16 * u);
-    }
-  };
-  auto mul = [&](int b) {
+  for (int d = 0; d < kRsAhead; d++)
+    if (d < nch) load(d, d);
+  for (int c0k = 0; c0k < nch; c0k += kRsAhead) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const float xs[8] = {xv[b][u][0].x, xv[b][u][0].y, xv[b][u][0].z, xv[b][u][0].w,
-                           xv[b][u][1].x, xv[b][u][1].y, xv[b][u][1].z, xv[b][u][1].w};
-      bf16x8 hi, lo;
+    for (int d = 0; d < kRsAhead; d++) {
+      const int c = c0k + d;
+      if (c >= nch) break;
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        hi[e] = (__bf16)xs[e];
-        lo[e] = (__bf16)(xs[e] - (float)hi[e]);
+      for (int i = 0; i < 4; i++) {
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          hi[e] = (__bf16)xr[d][i][e];
+          lo[e] = (__bf16)(xr[d][i][e] - (float)hi[e]);
+        }
+        const int at = ((lane >> 3) + 8 * i) * kRsPitch + 4 * (lane & 7);
+        *(bf16x4 *)(xh + at) = hi;
+        *(bf16x4 *)(xl + at) = lo;
       }
-      const bf16x8 wb = __builtin_bit_cast(bf16x8, wv[b & 1][u]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, wb, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, wb, acc, 0, 0, 0);
-    }
-  };
-  if (live) {
-    load(0, 0);
-    for (int k0 = 0; k0 < kn; k0 += 32 * U) {  // two batches per trip, so the buffer index stays compile-time
-      if (k0 + 16 * U < kn) load(1, k0 + 16 * U);
-      mul(0);
-      if (k0 + 32 * U < kn) load(0, k0 + 32 * U);
-      if (k0 + 16 * U < kn) mul(1);
+#pragma unroll
+      for (int i = 0; i < 2; i++) *(u32x4 *)(wl + ((lane >> 2) + 16 * i) * kRsPitch + 8 * (lane & 3)) = wr[d][i];
+      if (c + kRsAhead < nch) load(d, c + kRsAhead);
+      __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses run in order: its writes are seen by its reads
+#pragma unroll
+      for (int u = 0; u < kRsKc / 16; u++) {
+        const int at = m * kRsPitch + 16 * u + 8 * h;
+        const bf16x8 w = *(const bf16x8 *)(wl + at);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(xh + at), w, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(xl + at), w, acc, 0, 0, 0);
+      }
+      __builtin_amdgcn_wave_barrier();  // the next chunk's writes come after these reads
     }
   }
+  __syncthreads();  // every wave's stages are read: the partial sums take their place
 #pragma unroll
   for (int i = 0; i < 16; i++) red[wave][i][lane] = acc[i];
   __syncthreads();
-  for (int o = threadIdx.x; o < CT * 16 * 64; o += kRouterWaves * 64) {
-    const int c = o / (16 * 64), i = (o >> 6) & 15, l = o & 63;
+  for (int o = threadIdx.x; o < 16 * 64; o += kRouterWaves * 64) {
+    const int i = o >> 6, l = o & 63;
     float v = 0.f;
 #pragma unroll
-    for (int k = 0; k < KSP; k++) v += red[k * CT + c][i][l];
-    const int r = rt * 32 + 4 * (l >> 5) + (i & 3) + 8 * (i >> 2), cc = (blockIdx.y * CT + c) * 32 + (l & 31);
+    for (int k = 0; k < kRouterWaves; k++) v += red[k][i][l];
+    const int r = r0 + 4 * (l >> 5) + (i & 3) + 8 * (i >> 2), cc = c0 + (l & 31);
     if (r < a.R && cc < ncol) a.logits[(uint64_t)r * (a.ne + 1) + cc] = bf16_round(v);
   }
 }
 
-// Many rows: a workgroup covers 64 rows x 128 columns over the whole k range, wave (rb, ct) = wave (rb = wave / 4,
-// ct = wave % 4) one 32 x 32 tile. The x rows are shared by the four column waves, so the workgroup stages each
-// 64-wide k chunk of them once through LDS, already split into bf16 hi and lo (the conversion runs once per element
-// per workgroup, and the rows cross from L2 once); each wave streams its own router columns from memory one chunk
-// ahead. Same arithmetic as bat_router (hi and lo products summed in f32), one k order.
-constexpr int kRtKc = 64, kRtRows = 64, kRtPitch = kRtKc + 8;  // k chunk, rows, LDS row pitch in bf16 (conflict-free)
-__global__ __launch_bounds__(512, 2) void bat_router_rows(MoeArgs a, int ngroups) {
-  __shared__ __attribute__((aligned(16))) __bf16 xs[2][2][kRtRows * kRtPitch];  // [buffer][hi, lo]
+// Many rows: a workgroup covers 64 rows x 64 columns over the whole k range, wave (rb, cb) of 2 x 2 one 32 x 32 tile.
+// A 128-wide k chunk of the rows and of the router's columns is staged in LDS at a time, the rows split into bf16 hi and
+// lo on the way (once per workgroup), two further chunks' loads in flight: what bounds this product is their latency,
+// so small tiles (72 -> 144 workgroups at 1111 rows) and few, deep chunks: 37.6 -> 26 us there, 41 -> 35 us at 4096
+// rows, against 64 x 128 tiles with 64-wide chunks one ahead. Same arithmetic as bat_router (hi and lo products summed
+// in f32), one k order; a chunk whose lo parts are all zero (rows of bf16 values) leaves their products out, exact zeros.
+constexpr int kRtKc = 128, kRtTile = 64, kRtPitch = kRtKc + 8;  // k chunk, tile side, LDS row pitch in bf16
+constexpr size_t kRtLds = (size_t)3 * kRtTile * kRtPitch * 2 + 8;
+__global__ __launch_bounds__(256, 2) void bat_router_rows(MoeArgs a, int ngroups) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  __bf16 *xh = (__bf16 *)lds, *xl = xh + kRtTile * kRtPitch, *wl = xl + kRtTile * kRtPitch;
+  int *lowf = (int *)(wl + kRtTile * kRtPitch);  // [2], by the chunk's parity: some lo part is not zero
+  const int ncol = a.ne + a.has_sgate, ncg = (ncol + kRtTile - 1) / kRtTile;
   int item;
-  if (!xcd_item(ngroups * ((a.ne + a.has_sgate + 127) / 128), item)) return;
-  const int ncol = a.ne + a.has_sgate, ncg = (ncol + 127) / 128, rg = item / ncg, cg = item % ncg;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rb = wave >> 2, ct = cg * 4 + (wave & 3);
-  const int m = lane & 31, h = lane >> 5;
-  const bool live = ct * 32 < ncol;
-  // staging: thread t converts row t / 8, k [8 (t % 8), +8) of the chunk
-  const int srow = threadIdx.x >> 3, sk = (threadIdx.x & 7) * 8;
-  const float *xp = a.x + (uint64_t)min(rg * kRtRows + srow, a.R - 1) * a.hid + sk;
-  const uint16_t *wp = a.router + (uint64_t)min(ct * 32 + m, ncol - 1) * a.hid + 8 * h;
-  const int nch = a.hid / kRtKc;
-  float4 xr[2];
-  uint4 wv[2][kRtKc / 16];
-  auto load_x = [&](int c) {
-    xr[0] = *(const float4 *)(xp + c * kRtKc);
-    xr[1] = *(const float4 *)(xp + c * kRtKc + 4);
-  };
-  auto load_w = [&](int b, int c) {
+  if (!xcd_item(ngroups * ncg, item)) return;
+  const int r0 = item / ncg * kRtTile, c0 = item % ncg * kRtTile;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 31, h = lane >> 5;
+  const int rw = (wave >> 1) * 32, cw = (wave & 1) * 32, nch = a.hid / kRtKc;
+  // staging: thread t takes inputs 4 (t % 32) .. + 3 of rows t / 32 + 8 i, and 16 bytes of columns t / 16 + 16 i
+  constexpr int D = 2, XI = kRtTile / 8, WI = kRtTile / 16;
+  f32x4 xr[D][XI];
+  u32x4 wr[D][WI];
+  auto load = [&](int d, int c) {
 #pragma unroll
-    for (int u = 0; u < kRtKc / 16; u++) wv[b][u] = *(const uint4 *)(wp + c * kRtKc + 16 * u);
-  };
-  auto stage = [&](int b) {
-    const float v[8] = {xr[0].x, xr[0].y, xr[0].z, xr[0].w, xr[1].x, xr[1].y, xr[1].z, xr[1].w};
-    bf16x8 hi, lo;
+    for (int i = 0; i < XI; i++)
+      xr[d][i] = *(const f32x4 *)(a.x + (uint64_t)min(r0 + (tid >> 5) + 8 * i, a.R - 1) * a.hid + c * kRtKc +
+                                  4 * (tid & 31));
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      hi[e] = (__bf16)v[e];
-      lo[e] = (__bf16)(v[e] - (float)hi[e]);
-    }
-    *(bf16x8 *)&xs[b][0][srow * kRtPitch + sk] = hi;
-    *(bf16x8 *)&xs[b][1][srow * kRtPitch + sk] = lo;
+    for (int i = 0; i < WI; i++)
+      wr[d][i] = *(const u32x4 *)(a.router + (uint64_t)min(c0 + (tid >> 4) + 16 * i, ncol - 1) * a.hid + c * kRtKc +
+                                  8 * (tid & 15));
   };
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; i++) acc[i] = 0.f;
-  auto mul = [&](int b) {
-    const __bf16 *ph = &xs[b][0][(rb * 32 + m) * kRtPitch + 8 * h], *pl = &xs[b][1][(rb * 32 + m) * kRtPitch + 8 * h];
+  const __bf16 *ah = xh + (rw + m) * kRtPitch + 8 * h, *al = xl + (rw + m) * kRtPitch + 8 * h;
+  const __bf16 *bw = wl + (cw + m) * kRtPitch + 8 * h;
+  auto chunk = [&](int d, int c) {
+    uint32_t low = 0;  // the lo parts' bits
 #pragma unroll
-    for (int u = 0; u < kRtKc / 16; u++) {
-      const bf16x8 hi = *(const bf16x8 *)(ph + 16 * u), lo = *(const bf16x8 *)(pl + 16 * u);
-      const bf16x8 wb = __builtin_bit_cast(bf16x8, wv[b][u]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, wb, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, wb, acc, 0, 0, 0);
-    }
-  };
-  // chunk c: stage it (its x already in registers), request chunk c + 1, one barrier, multiply. The buffer written
-  // at chunk c + 1 was last read at chunk c - 1, before every wave passed chunk c's barrier.
-  load_x(0);
-  if (live) load_w(0, 0);
-  for (int c = 0; c < nch; c += 2) {
-    stage(0);
-    if (c + 1 < nch) {
-      load_x(c + 1);
-      if (live) load_w(1, c + 1);
-    }
-    __syncthreads();
-    if (live) mul(0);
-    if (c + 1 < nch) {
-      stage(1);
-      if (c + 2 < nch) {
-        load_x(c + 2);
-        if (live) load_w(0, c + 2);
+    for (int i = 0; i < XI; i++) {
+      bf16x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        hi[e] = (__bf16)xr[d][i][e];
+        lo[e] = (__bf16)(xr[d][i][e] - (float)hi[e]);
       }
-      __syncthreads();
-      if (live) mul(1);
+      const uint2 lb = __builtin_bit_cast(uint2, lo);
+      low |= lb.x | lb.y;
+      const int at = ((tid >> 5) + 8 * i) * kRtPitch + 4 * (tid & 31);
+      *(bf16x4 *)(xh + at) = hi;
+      *(bf16x4 *)(xl + at) = lo;
     }
+#pragma unroll
+    for (int i = 0; i < WI; i++) *(u32x4 *)(wl + ((tid >> 4) + 16 * i) * kRtPitch + 8 * (tid & 15)) = wr[d][i];
+    if (__any(low != 0) && lane == 0) lowf[c & 1] = 1;
+    __syncthreads();
+    const int any = __builtin_amdgcn_readfirstlane(lowf[c & 1]);
+    if (tid == 0) lowf[(c + 1) & 1] = 0;  // the next chunk's, written past the barrier below
+    if (c + D < nch) load(d, c + D);
+    if (any) {
+#pragma unroll
+      for (int u = 0; u < kRtKc / 16; u++) {
+        const bf16x8 w = *(const bf16x8 *)(bw + 16 * u);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(ah + 16 * u), w, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(al + 16 * u), w, acc, 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kRtKc / 16; u++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(ah + 16 * u), *(const bf16x8 *)(bw + 16 * u), acc,
+                                                      0, 0, 0);
+    }
+    __syncthreads();  // the chunk's LDS is read
+  };
+  if (tid == 0) lowf[0] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < D; d++)
+    if (d < nch) load(d, d);
+  for (int c = 0; c < nch; c += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++)
+      if (c + d < nch) chunk(d, c + d);
   }
-  if (!live) return;
-  const int cc = ct * 32 + m;
+  const int cc = c0 + cw + m;
 #pragma unroll
   for (int i = 0; i < 16; i++) {
-    const int r = rg * kRtRows + rb * 32 + 4 * h + (i & 3) + 8 * (i >> 2);
+    const int r = r0 + rw + 4 * h + (i & 3) + 8 * (i >> 2);
     if (r < a.R && cc < ncol) a.logits[(uint64_t)r * (a.ne + 1) + cc] = bf16_round(acc[i]);
   }
 }
@@ -1655,6 +1676,7 @@ static void gemm_attrs_all() {
   gemm_attrs<K, KS, true, 64>();
 }
 void init_batch_attrs() {
+  IJ_HIP(hipFuncSetAttribute((const void *)&bat_router_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRtLds));
   init_q8_attrs();
   IJ_HIP(hipFuncSetAttribute((const void *)&bat_place_prep, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPrepLds));
   gemm_attrs_all<4, 4>(); gemm_attrs_all<5, 5>(); gemm_attrs_all<6, 6>(); gemm_attrs_all<4, 5>();
@@ -1714,8 +1736,9 @@ int moe_batch_max_chunks(int R, int ne, int topk, bool shared) {
 void launch_moe_batch(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
   const int ncol = a.ne + a.has_sgate, S = a.R * a.nslot;
   if (a.R >= 512) {
-    const int ng = (a.R + kRtRows - 1) / kRtRows;
-    hipLaunchKernelGGL(bat_router_rows, dim3((ng * ((ncol + 127) / 128) + 7) & ~7), dim3(512), 0, s, a, ng);
+    const int ng = (a.R + kRtTile - 1) / kRtTile;
+    hipLaunchKernelGGL(bat_router_rows, dim3((ng * ((ncol + kRtTile - 1) / kRtTile) + 7) & ~7), dim3(256), kRtLds, s, a,
+                       ng);
   } else if (moe_batch_exact(a)) {
     IJ_CHECK(a.hid / 512 <= kRouterExactChunks, "few-row router: hidden %d above %d", a.hid, 512 * kRouterExactChunks);
     const int nc = a.hid / 512;
@@ -1726,7 +1749,7 @@ void launch_moe_batch(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
     else
       hipLaunchKernelGGL(bat_router_exact<kRouterExactChunks>, dim3((ncol + 3) / 4, a.R), dim3(256), 0, s, a);
   } else {
-    hipLaunchKernelGGL(bat_router<1>, dim3((a.R + 31) / 32, (ncol + 31) / 32), dim3(64 * kRouterWaves), 0, s, a);
+    hipLaunchKernelGGL(bat_router, dim3((a.R + 31) / 32, (ncol + 31) / 32), dim3(64 * kRouterWaves), 0, s, a);
   }
   const int KS = a.nslot > a.topk ? a.slay.K : a.lay.K;
   const bool few = moe_batch_exact(a) && b.vpart && moe_batch_few(a.R, a.hid, a.inter, a.lay.K, KS);
