@@ -1030,9 +1030,10 @@ __device__ __forceinline__ void h32_operand(int lane, J jmap, f16x8 (&hA)[2]) {
 __device__ __forceinline__ f32x16 h32_tile(const f32x16 &v, const f16x8 (&hA)[2], int lane) {
   float mx = 0.f;
 #pragma unroll
-  for (int i = 0; i < 16; i++) mx = fmaxf(mx, fabsf(v[i]));
+  for (int i = 0; i < 16; i += 2) mx = fmaxf(fmaxf(mx, fabsf(v[i])), fabsf(v[i + 1]));
   mx = fmaxf(mx, xor_lane<32>(mx, lane));
   const int ex = min(max(141 - (int)((__float_as_uint(mx) >> 23) & 0xFFu), -126), 127);
+  const float up = __builtin_ldexpf(1.f, ex), down = __builtin_ldexpf(1.f, -ex);  // powers of two: exact products
   f32x16 T;
 #pragma unroll
   for (int i = 0; i < 16; i++) T[i] = 0.f;
@@ -1041,16 +1042,24 @@ __device__ __forceinline__ f32x16 h32_tile(const f32x16 &v, const f16x8 (&hA)[2]
     f16x8 hi, lo;
 #pragma unroll
     for (int t = 0; t < 8; t++) {
-      const float w = __builtin_ldexpf(v[8 * st + t], ex);
+      const float w = v[8 * st + t] * up;
       hi[t] = (_Float16)w;
-      lo[t] = (_Float16)(w - (float)hi[t]);
+      lo[t] = (_Float16)__builtin_fmaf((float)hi[t], -1.f, w);
     }
     T = __builtin_amdgcn_mfma_f32_32x32x16_f16(hA[st], hi, T, 0, 0, 0);
     T = __builtin_amdgcn_mfma_f32_32x32x16_f16(hA[st], lo, T, 0, 0, 0);
   }
 #pragma unroll
-  for (int i = 0; i < 16; i++) T[i] = __builtin_ldexpf(T[i], -ex);
+  for (int i = 0; i < 16; i++) T[i] = T[i] * down;
   return T;
+}
+// H_4 over the four chunks of a 128-block: t[q] -> sum over q' of (-1)^popcount(q & q') t[q']
+__device__ __forceinline__ void h4(float (&t)[4]) {
+  const float a0 = t[0] + t[1], a1 = t[0] - t[1], a2 = t[2] + t[3], a3 = t[2] - t[3];
+  t[0] = a0 + a2;
+  t[1] = a1 + a3;
+  t[2] = a0 - a2;
+  t[3] = a1 - a3;
 }
 
 // EX (few rows, speculative verify): the one-row step's arithmetic throughout, so that every row is bit-identical
@@ -1126,22 +1135,28 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
   } else {
   // epilogue per 32-row block, with the tiles transposed (wave w: projection w / 4, chunk q = w % 4 of block ib):
   //  1. every wave: H_32 on its tile (element j = 8 (i / 4) + 4 h + i % 4 at lane (n, h) value i), tile to LDS;
-  //  2. waves 0..3 (chunk q): H_4 over the gate tiles and over the up tiles gives g and u of columns 32 q + j; then
-  //     h = silu(g svh_g / sqrt(128)) u svh_u / sqrt(128) suh_d, already in the layout of a tile, and H_32 on it
-  //     with the rows in kp order (lane (n, h) value i = kp position 16 h + i of the chunk), to LDS;
-  //  3. wave w takes rows 4 w .. 4 w + 3 whole: lane l combines kp positions 2 l, 2 l + 1 with H_4, / sqrt(128), and
-  //     each row leaves as one 256-byte store.
+  //  2. every wave: elements 4 w + 2 h, + 1 of all four chunks of row n: H_4 over the gate and the up tiles gives g and u,
+  //     h = silu(g svh_g / sqrt(128)) u svh_u / sqrt(128) suh_d, H_4 on it, back to LDS as four tiles;
+  //  3. waves 0..3 (chunk q): H_32 with the rows in kp order: lane (n, h) holds kp positions 16 h .. 16 h + 15 of its row's
+  //     chunk and stores them, 32 bytes.
+  // (With H_4 as one of four outputs per lane, four multiply-adds per value on half the waves, and the H_4 of the last
+  // step read whole rows from LDS again, the epilogues were 25% of the vector instructions here and 44% in bat_down.)
   const int q = wave & 3, n = lane & 31, h = lane >> 5;
   f16x8 hA1[2], hA2[2];
   h32_operand(lane, [](uint32_t m) { return m; }, hA1);
   h32_operand(lane, [](uint32_t m) { return kp_inv32(16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u)); }, hA2);
-  // scales of this lane's columns in step 2: 32 q + 8 g + 4 h + r (natural order inside block ib), read per block
-  const int c0 = ib * 128 + 32 * q + 4 * h;
-  const uint16_t *pg = (const uint16_t *)(blk + sv_of(a, e, 0)) + c0, *pu = (const uint16_t *)(blk + sv_of(a, e, 1)) + c0;
-  const uint16_t *pd = (const uint16_t *)(blk + su_of(a, e, 2)) + c0;
+  const int e0 = 4 * wave + 2 * h;  // step 2's elements
   const float sc = a.sc_inter;
+  f16x2 sg[4], su[4], sd[4];  // their scales: columns 32 c + e0, + 1 of block ib
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const int col = ib * 128 + 32 * c + e0;
+    sg[c] = *(const f16x2 *)((const uint16_t *)(blk + sv_of(a, e, 0)) + col);
+    su[c] = *(const f16x2 *)((const uint16_t *)(blk + sv_of(a, e, 1)) + col);
+    sd[c] = *(const f16x2 *)((const uint16_t *)(blk + su_of(a, e, 2)) + col);
+  }
   // LDS: 8 step-1 tiles of 32 rows x 32 elements, row pitch 36 floats; the 4 step-2 tiles take their place
-  float *x1 = (float *)lds, *x2 = x1;
+  float *xt = (float *)lds;
   const int nrb = (nrows + 31) / 32;
 #pragma unroll
   for (int rb = 0; rb < NRB; rb++) {
@@ -1150,61 +1165,56 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
     __syncthreads();  // the ring (first block) or the previous block's tiles are no longer read
 #pragma unroll
     for (int g = 0; g < 4; g++)
-      *(float4 *)(x1 + (wave * 32 + n) * 36 + 8 * g + 4 * h) = make_float4(T[4 * g], T[4 * g + 1], T[4 * g + 2], T[4 * g + 3]);
+      *(float4 *)(xt + (wave * 32 + n) * 36 + 8 * g + 4 * h) = make_float4(T[4 * g], T[4 * g + 1], T[4 * g + 2], T[4 * g + 3]);
     __syncthreads();
-    f32x16 T2;
-    if (wave < 4) {
-      f32x16 hv;
+    float hv[2][4];  // [element][chunk]
+    {
+      float g[2][4], u[2][4];
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const f16x4 sgv = *(const f16x4 *)(pg + 8 * g), suv = *(const f16x4 *)(pu + 8 * g), sdv = *(const f16x4 *)(pd + 8 * g);
-        float4 gs = {0.f, 0.f, 0.f, 0.f}, us = gs;
-#pragma unroll
-        for (int qq = 0; qq < 4; qq++) {
-          const float sgn = (__builtin_popcount(q & qq) & 1) ? -1.f : 1.f;
-          const float4 tg = *(const float4 *)(x1 + (qq * 32 + n) * 36 + 8 * g + 4 * h);
-          const float4 tu = *(const float4 *)(x1 + ((4 + qq) * 32 + n) * 36 + 8 * g + 4 * h);
-          gs.x = __builtin_fmaf(sgn, tg.x, gs.x);
-          gs.y = __builtin_fmaf(sgn, tg.y, gs.y);
-          gs.z = __builtin_fmaf(sgn, tg.z, gs.z);
-          gs.w = __builtin_fmaf(sgn, tg.w, gs.w);
-          us.x = __builtin_fmaf(sgn, tu.x, us.x);
-          us.y = __builtin_fmaf(sgn, tu.y, us.y);
-          us.z = __builtin_fmaf(sgn, tu.z, us.z);
-          us.w = __builtin_fmaf(sgn, tu.w, us.w);
-        }
-        const float gv[4] = {gs.x, gs.y, gs.z, gs.w}, uv[4] = {us.x, us.y, us.z, us.w};
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const float gg = gv[r] * sc * (float)sgv[r], uu = uv[r] * sc * (float)suv[r];
-          // SiLU with the hardware exp2 and reciprocal (~1 ulp each; the layer's tolerance is 1e-2)
-          hv[4 * g + r] = gg * __builtin_amdgcn_rcpf(1.f + __expf(-gg)) * uu * (float)sdv[r];
-        }
+      for (int c = 0; c < 4; c++) {
+        const float2 tg = *(const float2 *)(xt + (c * 32 + n) * 36 + e0), tu = *(const float2 *)(xt + ((4 + c) * 32 + n) * 36 + e0);
+        g[0][c] = tg.x;
+        g[1][c] = tg.y;
+        u[0][c] = tu.x;
+        u[1][c] = tu.y;
       }
-      T2 = h32_tile(hv, hA2, lane);
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        h4(g[t]);
+        h4(u[t]);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const float gg = g[t][c] * sc * (float)sg[c][t], uu = u[t][c] * sc * (float)su[c][t];
+          // SiLU with the hardware exp2 and reciprocal (~1 ulp each; the layer's tolerance is 1e-2)
+          hv[t][c] = gg * __builtin_amdgcn_rcpf(1.f + __expf(-gg)) * uu * (float)sd[c][t];
+        }
+        h4(hv[t]);
+      }
     }
     __syncthreads();  // the step-1 tiles are read
-    if (wave < 4) {
 #pragma unroll
-      for (int g = 0; g < 4; g++)
-        *(float4 *)(x2 + (q * 32 + n) * 36 + 16 * h + 4 * g) = make_float4(T2[4 * g], T2[4 * g + 1], T2[4 * g + 2], T2[4 * g + 3]);
-    }
+    for (int c = 0; c < 4; c++) *(float2 *)(xt + (c * 32 + n) * 36 + e0) = make_float2(hv[0][c], hv[1][c]);
     __syncthreads();
-    const int oq = lane >> 4, op = 2 * (lane & 15);  // this lane's kp positions 32 oq + op, + 1
+    if (wave < 4) {
+      f32x16 v;
 #pragma unroll
-    for (int rr = 0; rr < 4; rr++) {
-      const int nr = wave * 4 + rr, r = rb * 32 + nr;
-      if (r >= nrows) break;
-      float o0 = 0.f, o1 = 0.f;
-#pragma unroll
-      for (int qq = 0; qq < 4; qq++) {
-        const float sgn = (__builtin_popcount(oq & qq) & 1) ? -1.f : 1.f;
-        const float2 t = *(const float2 *)(x2 + (qq * 32 + nr) * 36 + op);
-        o0 = __builtin_fmaf(sgn, t.x, o0);
-        o1 = __builtin_fmaf(sgn, t.y, o1);
+      for (int g = 0; g < 4; g++) {
+        const float4 t = *(const float4 *)(xt + (q * 32 + n) * 36 + 8 * g + 4 * h);
+        v[4 * g] = t.x;
+        v[4 * g + 1] = t.y;
+        v[4 * g + 2] = t.z;
+        v[4 * g + 3] = t.w;
       }
-      *(uint32_t *)(hh + (uint64_t)(row0 + r) * a.inter + ib * 128 + 2 * lane) =
-          __builtin_bit_cast(uint32_t, f16x2{(_Float16)(o0 * sc), (_Float16)(o1 * sc)});
+      const f32x16 T2 = h32_tile(v, hA2, lane);
+      const int r = rb * 32 + n;
+      f16x8 o[2];
+#pragma unroll
+      for (int i = 0; i < 16; i++) o[i >> 3][i & 7] = (_Float16)(T2[i] * sc);
+      if (r < nrows) {
+        f16x8 *out = (f16x8 *)(hh + (uint64_t)(row0 + r) * a.inter + ib * 128 + 32 * q + 16 * h);
+        out[0] = o[0];
+        out[1] = o[1];
+      }
     }
   }
   }
@@ -1276,17 +1286,15 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
   } else {
   // epilogue: wave w holds columns 32 w .. of this 256 (block bb = w / 4, chunk q = w % 4) for every row, transposed.
   // Per 32-row block: H_32 on the wave's tile (output element j = 16 h + i of the chunk at lane (n, h)), the tiles to
-  // LDS; then wave w takes rows 4 w .. 4 w + 3 whole: lane l combines columns 4 l .. 4 l + 3 with H_4 across the four
-  // chunks of its block, applies 1/sqrt(128), svh_d and the slot's route weight, and the row leaves as one 1 KB store.
+  // LDS; then wave w takes rows 4 w .. 4 w + 3 whole: lane (element j, block bb) reads its element of the block's four
+  // chunks, and H_4 gives it the row's four columns 32 q + j, times 1/sqrt(128), svh_d and the slot's route weight.
   f16x8 hA[2];
   h32_operand(lane, [](uint32_t m) { return 16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u); }, hA);
-  const int cb = lane >> 5, cq = (lane >> 3) & 3, cj = 4 * (lane & 7);  // this lane's columns: block, chunk, element
+  const int cb = lane >> 5, cj = lane & 31;
   float sv[4];
-  {
-    const uint16_t *svp = (const uint16_t *)(blk + sv_of(a, e, 2)) + ob2 * 256 + 4 * lane;
 #pragma unroll
-    for (int t = 0; t < 4; t++) sv[t] = h2f(svp[t]) * a.sc_hid;
-  }
+  for (int t = 0; t < 4; t++)
+    sv[t] = h2f(((const uint16_t *)(blk + sv_of(a, e, 2)))[ob2 * 256 + cb * 128 + 32 * t + cj]) * a.sc_hid;
   // 8 tiles of 32 rows x 32 columns: tile w, row n, element j at (w 32 + n) 36 + j floats (the pad spreads the
   // rows of one write over the banks)
   float *xt = (float *)lds;
@@ -1306,19 +1314,14 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
     for (int rr = 0; rr < 4; rr++) {
       const int n = wave * 4 + rr, r = rb * 32 + n;
       if (r >= nrows) break;
-      float4 o = {0.f, 0.f, 0.f, 0.f};
+      float t[4];
 #pragma unroll
-      for (int qq = 0; qq < 4; qq++) {
-        const float4 t = *(const float4 *)(xt + ((cb * 4 + qq) * 32 + n) * 36 + cj);
-        const float sg = (__builtin_popcount(cq & qq) & 1) ? -1.f : 1.f;
-        o.x = __builtin_fmaf(sg, t.x, o.x);
-        o.y = __builtin_fmaf(sg, t.y, o.y);
-        o.z = __builtin_fmaf(sg, t.z, o.z);
-        o.w = __builtin_fmaf(sg, t.w, o.w);
-      }
+      for (int qq = 0; qq < 4; qq++) t[qq] = xt[((cb * 4 + qq) * 32 + n) * 36 + cj];
+      h4(t);
       const float w = m_w[r];
-      *(float4 *)(dnw + (uint64_t)m_dst[r] * a.hid + ob2 * 256 + 4 * lane) =  // slot = token nslot + k
-          make_float4(o.x * sv[0] * w, o.y * sv[1] * w, o.z * sv[2] * w, o.w * sv[3] * w);
+      float *out = dnw + (uint64_t)m_dst[r] * a.hid + ob2 * 256 + cb * 128 + cj;  // slot = token nslot + k
+#pragma unroll
+      for (int qq = 0; qq < 4; qq++) out[32 * qq] = t[qq] * sv[qq] * w;
     }
   }
   }
