@@ -613,8 +613,10 @@ struct ne_moe {
   void ensure_batch(int R) {
     if (R <= bat_R || !batch_ok(R)) return;
     free_batch();
-    if (moe_batch_few(R, hid, inter, K, has_shared ? Ks : K)) {
-      bat.vmax_chunks = moe_batch_few_chunks(R, ne, topk, has_shared);
+    // (buffers sized for many rows serve the few-row calls too: without the pool those would leave their path)
+    const int few = std::min(R, 32);
+    if (moe_batch_few(few, hid, inter, K, has_shared ? Ks : K)) {
+      bat.vmax_chunks = moe_batch_few_chunks(few, ne, topk, has_shared);
       few_pool(hid, inter, bat.vmax_chunks, &bat.vpart, &bat.vep);
     }
     const size_t S = (size_t)R * nslot();

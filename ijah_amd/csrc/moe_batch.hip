@@ -1638,10 +1638,12 @@ void launch_few_rt(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
   constexpr int KM = K > KS ? K : KS;
   const int NBI = a.inter / 128, NBLK = a.hid / 128;
   const size_t lg = v_gu_lds<KM, RT>(a.hid / 512), ld = v_dn_lds<KM, RT>(a.inter);
-  hipLaunchKernelGGL((bat_gu_grp<K, KS, RT>), dim3(b.vmax_chunks * NBI * 8), dim3(256), lg, s, a, b.bk, b.chunks,
-                     b.xh, b.hh, b.vpart, b.vep);
-  hipLaunchKernelGGL((bat_dn_blk<K, KS, RT>), dim3(b.vmax_chunks * NBLK), dim3(256), ld, s, a, b.bk, b.chunks, b.rows,
-                     b.hh, b.dnw);
+  // the grid of this row count (the pool may hold more: 32 rows' chunks, 2 rows' launch would start 12000 idle workgroups)
+  const int most = moe_batch_few_chunks(a.R, a.ne, a.topk, a.nslot > a.topk);
+  hipLaunchKernelGGL((bat_gu_grp<K, KS, RT>), dim3(most * NBI * 8), dim3(256), lg, s, a, b.bk, b.chunks, b.xh, b.hh,
+                     b.vpart, b.vep);
+  hipLaunchKernelGGL((bat_dn_blk<K, KS, RT>), dim3(most * NBLK), dim3(256), ld, s, a, b.bk, b.chunks, b.rows, b.hh,
+                     b.dnw);
 }
 template <int K, int KS>
 void launch_few(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {

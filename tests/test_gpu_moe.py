@@ -590,3 +590,17 @@ def test_moe_q8_many_rows_tiles(eng, hid, inter, R, whole):
     g, u = lin("gate", x.astype(np.float64), inter, hid), lin("up", x.astype(np.float64), inter, hid)
     want = lin("down", _rr(g / (1 + np.exp(-g)) * u), hid, inter)
     assert rel(m.read("shared_q8", R), want) < 1e-3
+
+
+def test_moe_few_rows_after_many(eng):
+    """A layer whose buffers a many-row run sized keeps the few-row path (and its bits), at a row count below the largest
+    the shared pool has served."""
+    w = synth.moe_layer(970, hid=1024, inter=256, ne=32, topk=4, K=5, shared=True, Ks=5)
+    rng = np.random.default_rng(971)
+    x = synth.bf16_values(rng, 300, 1024)
+    first, later = eng.moe_create(w), eng.moe_create(w)
+    want = {R: first.run(x[:R]) for R in (1, 5, 32)}
+    later.run(x)
+    for R in (32, 5, 2, 1):
+        got = later.run(x[:R])
+        assert np.array_equal(got, want[R] if R in want else want[5][:R]), R
