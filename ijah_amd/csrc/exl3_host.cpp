@@ -58,7 +58,7 @@ struct ne_exl3_lin {
   uint32_t *tiles = nullptr;
   uint16_t *suh = nullptr, *svh = nullptr;
   uint16_t *xh = nullptr;  // [kLinMaxRows][in]
-  float *part = nullptr;   // [S][part_rows][OTp*16]: k group partials
+  float *part = nullptr;   // [groups()][part_rows][OTp*16]: k group partials
   uint32_t *cnt = nullptr; // per 128-column output block (the one-launch path's completion counters)
   bool one_launch = true;  // IJAH_LIN_PATH=staged at creation: prep, GEMM and finish as three launches
   int part_rows = 0;
@@ -220,7 +220,8 @@ static LinArgs lin_args(ne_exl3_lin *l, int R, const float *x, float *y, const L
     IJ_HIP(hipStreamIsCapturing(stream(), &cs));
     IJ_CHECK(cs == hipStreamCaptureStatusNone, "linear: partial scratch must grow before a stream capture");
     dev_free(l->part);
-    l->part = dev_alloc<float>((size_t)S * R * l->OTp * 16);
+    // (room for every k group at any S: the paths that store fewer may be switched to one that stores them all)
+    l->part = dev_alloc<float>((size_t)l->groups() * R * l->OTp * 16);
     l->part_rows = R;
   }
   LinArgs a;

@@ -6,6 +6,7 @@
 //   - allocates, frees, sets memory, changes a kernel attribute or waits on a stream while a stream is capturing;
 //   - frees memory that a live captured graph (or graph exec) still references;
 //   - launches (eagerly or by replaying a graph) a kernel whose arguments point into freed memory;
+//   - launches a linear whose k group partials or prepared rows are more than the memory they point to holds;
 //   - destroys a graph exec while replays are notionally still running (a replay not followed by a wait).
 // The launchers record the device pointers of their argument structs (LinArgs, MoeArgs), so a captured graph knows
 // every buffer it will read or write.
@@ -70,6 +71,13 @@ void use(const void *ptr, const char *kernel) {
   if (it == allocs.end()) return;  // not device memory the stand-in made (e.g. a host scalar): not tracked
   if (!it->second.live) violation("%s: argument %p points into freed memory", kernel, ptr);
   if (capturing) cap.uses.insert(it->first);
+}
+// the kernel writes `bytes` from ptr on: they must fit the allocation
+void room(const void *ptr, size_t bytes, const char *kernel, const char *what) {
+  const uintptr_t p = (uintptr_t)ptr;
+  auto it = ptr ? find_alloc(p) : allocs.end();
+  if (it != allocs.end() && p + bytes > it->first + it->second.n)
+    violation("%s: %s takes %zu bytes, room for %zu", kernel, what, bytes, (size_t)(it->first + it->second.n - p));
 }
 void check_graph(const Graph &g, const char *what) {
   for (uintptr_t b : g.uses) {
@@ -314,6 +322,8 @@ static void use_lin(const LinArgs &a, const char *k) {
                         (const void *)a.epi.e0, (const void *)a.epi.e1, (const void *)a.epi.e2, (const void *)a.epi.e3,
                         (const void *)a.epi.e4, (const void *)a.epi.w16, (const void *)a.epi.ctr})
     use(p, k);
+  room(a.part, (size_t)a.S * a.R * (a.OT + (a.OT & 1)) * 16 * 4, k, "partials");
+  if (a.xh_in) room(a.xh, (size_t)a.R * a.in * 2, k, "prepared rows");
 }
 void launch_lin(const LinArgs &a, hipStream_t) {
   std::lock_guard<std::recursive_mutex> l(mu);

@@ -126,6 +126,20 @@ def test_linear_refuses_growth_under_capture(host):
     clean(eng)
 
 
+@pytest.mark.parametrize("R", [1, 4])
+def test_partials_hold_the_staged_path_after_the_loop(host, R):
+    """a vocabulary-wide linear at few rows keeps one total per column (its workgroups loop over the k groups); switched
+    to the staged path afterwards it stores every k group's partials, at the same row count"""
+    eng = host
+    eng.lib.hipstub_reset()
+    lin = linears(eng, [(2048, 65536, 2)], seed=3)[0]
+    x, y = eng.alloc(R * 2048 * 4), eng.alloc(R * 65536 * 4)
+    lin.run_bufs(R, x, y)
+    lin.configure("staged", 1)
+    lin.run_bufs(R, x, y)
+    clean(eng)
+
+
 def test_instrumentation_sees_violations(host):
     """the stand-in reports an allocation inside a capture and a buffer freed while a live graph exec uses it"""
     eng = host
