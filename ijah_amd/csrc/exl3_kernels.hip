@@ -613,15 +613,15 @@ __global__ __launch_bounds__(64) void lin_prep(LinArgs a) {
 // epilogue (reference kernels/trunk6/trunk6.metal:199-214, t6_finish). coherent: the partials were stored by other
 // workgroups of this launch (device-coherent loads); else by an earlier launch.
 // Rows r0, r0 + rs, .. (NR of them, those below R) of output block cb: each row's k-group partials folded left in
-// group order, H_out, svh and the epilogue. The partials of all NR rows are requested together, up to BMAX groups at a
-// time, so a wave finishing several rows pays one round trip per round, not one per row. sv: the lane's svh of the block
-// (lin_svh).
+// group order, H_out, svh and the epilogue. The partials of all NR rows are requested together, in rounds of groups, so
+// a wave finishing several rows pays one round trip per round, not one per row: rounds of 4 groups for several rows, of
+// 8 for one, or of B1 where there are more than 8. sv: the lane's svh of the block (lin_svh).
 __device__ __forceinline__ void lin_svh(const LinArgs &a, int cb, uint16_t (&sv)[2]) {
   const int i0 = cb * 128 + (threadIdx.x & 63), i1 = i0 + 64;
   sv[0] = a.svh[i0 < a.out ? i0 : 0];
   sv[1] = a.svh[i1 < a.out ? i1 : 0];
 }
-template <int NR, int BMAX>
+template <int NR, int B1 = 8>
 __device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool coherent, const uint16_t (&sv)[2]) {
   const int lane = threadIdx.x & 63, OTp = a.OT + (a.OT & 1);
   const int i0 = cb * 128 + lane, i1 = i0 + 64;
@@ -630,33 +630,35 @@ __device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool c
   float v0[NR], v1[NR];
 #pragma unroll
   for (int q = 0; q < NR; q++) v0[q] = v1[q] = 0.f;
-  auto fold = [&](auto bc, int g0) {  // groups g0 .. g0 + B - 1 (those below S)
+  auto fold = [&](auto bc) {  // rounds of B groups
     constexpr int B = decltype(bc)::value;
-    float t0[NR][B], t1[NR][B];
+    for (int g0 = 0; g0 < a.S; g0 += B) {
+      float t0[NR][B], t1[NR][B];
 #pragma unroll
-    for (int q = 0; q < NR; q++) {
-      const int r = min(r0 + q * rs, a.R - 1);
+      for (int q = 0; q < NR; q++) {
+        const int r = min(r0 + q * rs, a.R - 1);
 #pragma unroll
-      for (int j = 0; j < B; j++) {
-        const float *pp = a.part + ((uint64_t)min(g0 + j, a.S - 1) * a.R + r) * OTp * 16;
-        t0[q][j] = coherent ? ld_cg(pp + j0) : pp[j0];
-        t1[q][j] = coherent ? ld_cg(pp + j1) : pp[j1];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < NR; q++)
-#pragma unroll
-      for (int j = 0; j < B; j++)
-        if (g0 + j < a.S) {
-          v0[q] = g0 + j == 0 ? t0[q][j] : v0[q] + t0[q][j];
-          v1[q] = g0 + j == 0 ? t1[q][j] : v1[q] + t1[q][j];
+        for (int j = 0; j < B; j++) {
+          const float *pp = a.part + ((uint64_t)min(g0 + j, a.S - 1) * a.R + r) * OTp * 16;
+          t0[q][j] = coherent ? ld_cg(pp + j0) : pp[j0];
+          t1[q][j] = coherent ? ld_cg(pp + j1) : pp[j1];
         }
+      }
+#pragma unroll
+      for (int q = 0; q < NR; q++)
+#pragma unroll
+        for (int j = 0; j < B; j++)
+          if (g0 + j < a.S) {
+            v0[q] = g0 + j == 0 ? t0[q][j] : v0[q] + t0[q][j];
+            v1[q] = g0 + j == 0 ? t1[q][j] : v1[q] + t1[q][j];
+          }
+    }
   };
   constexpr int kFew = NR == 1 ? 8 : 4;
-  if (a.S <= kFew)
-    fold(std::integral_constant<int, kFew>{}, 0);
+  if (NR > 1 || B1 == kFew || a.S <= kFew)
+    fold(std::integral_constant<int, kFew>{});
   else
-    for (int g0 = 0; g0 < a.S; g0 += BMAX) fold(std::integral_constant<int, BMAX>{}, g0);
+    fold(std::integral_constant<int, B1>{});
 #pragma unroll
   for (int q = 0; q < NR; q++) {
     const int r = r0 + q * rs;
@@ -670,16 +672,15 @@ __device__ void lin_finish_rows(const LinArgs &a, int r0, int rs, int cb, bool c
 __device__ void lin_finish_row(const LinArgs &a, int r, int cb, bool coherent) {
   uint16_t sv[2];
   lin_svh(a, cb, sv);
-  lin_finish_rows<1, 8>(a, r, 1, cb, coherent, sv);
+  lin_finish_rows<1>(a, r, 1, cb, coherent, sv);
 }
-// the block's rows over the workgroup's 4 waves (wave c: rows c, c + 4, ..), four rows per request round; B1 and B4: the
-// groups per round for one row and for four
-template <int B1, int B4>
+// the block's rows over the workgroup's 4 waves (wave c: rows c, c + 4, ..), four rows per request round
+template <int B1 = 8>
 __device__ void lin_finish_block(const LinArgs &a, int c, int cb, const uint16_t (&sv)[2]) {
   if (a.R <= 4) {
     if (c < a.R) lin_finish_rows<1, B1>(a, c, 4, cb, true, sv);
   } else {
-    for (int r = c; r < a.R; r += 16) lin_finish_rows<4, B4>(a, r, 4, cb, true, sv);
+    for (int r = c; r < a.R; r += 16) lin_finish_rows<4>(a, r, 4, cb, true, sv);
   }
 }
 
@@ -727,11 +728,12 @@ __global__ __launch_bounds__(256) void lin_mx(LinMulti m) {
   float *csum = (float *)(lds + 4 * lin_wave_lds<K, RT>());  // [4 chunks][RT rows][32 columns]
   const int e0 = kt0 * 16, i0 = e0 + lane, i1 = i0 + 64;    // the chunk's elements of this lane
   const int cb = p / 4;
-  // The finisher's svh is requested with the first loads, so that its latency is not paid after the hand-off, and the
-  // partials of up to 24 k groups (the reference's trunk has 20) in one round: up to 16 rows these small launches are
-  // chains of round trips (q, k, v and o of eight layers at one row 143 -> 133 us, the HC read of eight 153 -> 146). At 32
-  // rows, and in the kernels with many workgroups per output block, the registers cost more than the round trips
-  // (170 -> 178 us; vocabulary head at one row 82 -> 87): there svh is loaded late and the rounds are shorter.
+  // The finisher's svh is requested with the first loads, so that its latency is not paid after the hand-off: up to 16
+  // rows these small launches are chains of round trips. One row's partials come in rounds of 12 k groups (the
+  // reference's trunk has 20): any more registers cost all workgroups a wave per SIMD, for the one per output block that
+  // finishes. Rounds of 24, with three waves per SIMD instead of four, were no faster where the grid fits the chip at
+  // once (2048 -> 4096 K6 at one row 7.9 us, both) and slower where it does not (2560 -> 10240 15.4 us, 14.2 with 12;
+  // 4096 -> 16384 K5 24.6 and 22.0). At 32 rows svh is loaded late: requesting it first cost more (170 -> 178 us).
   uint16_t sv[2];
   if constexpr (RT < 32) lin_svh(a, cb, sv);
   // 1. input rows and tiles
@@ -869,7 +871,7 @@ __global__ __launch_bounds__(256) void lin_mx(LinMulti m) {
   if (block_signal(ctr, &flag) != (uint32_t)(npb * a.S - 1)) return;
   if (threadIdx.x == 0) st_cg(ctr, 0u);
   if constexpr (RT >= 32) lin_svh(a, cb, sv);
-  lin_finish_block<(RT <= 4 ? 24 : 8), (RT < 32 ? 8 : 4)>(a, c, cb, sv);
+  lin_finish_block<(RT <= 4 ? 12 : 8)>(a, c, cb, sv);
   if (a.epi.kind == 8)
     hc_fin_block(a, a.epi.ctr + (uint64_t)(cb % (a.epi.hid / 128)) * kSyncStride, a.epi.row0, a.epi.row0 + R, cb,
                  &flag);
@@ -956,7 +958,7 @@ __global__ __launch_bounds__(256) void lin_mxl(LinMulti m) {
   if (threadIdx.x == 0) st_cg(ctr, 0u);
   uint16_t sv[2];
   lin_svh(a, cb, sv);
-  lin_finish_block<8, 4>(a, c, cb, sv);
+  lin_finish_block(a, c, cb, sv);
   if (a.epi.kind == 8)
     hc_fin_block(a, a.epi.ctr + (uint64_t)(cb % (a.epi.hid / 128)) * kSyncStride, a.epi.row0, a.epi.row0 + R, cb,
                  &flag);
@@ -1049,7 +1051,7 @@ __global__ __launch_bounds__(64 * NW) void lin_mxw(LinMulti m) {
   if (last & (1u << b)) {
     uint16_t sv[2];
     lin_svh(a, (NW / 4) * bp + b, sv);
-    lin_finish_block<8, 4>(a, w & 3, (NW / 4) * bp + b, sv);
+    lin_finish_block(a, w & 3, (NW / 4) * bp + b, sv);
   }
 }
 

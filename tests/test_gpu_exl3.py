@@ -104,6 +104,25 @@ def test_linear_rows_bit_identical(eng, oracle, inp, out, K, R):
     assert np.array_equal(lin.run(x[:3]), y[:3])
 
 
+@pytest.mark.parametrize("inp,out,K", [(6144, 128, 4), (6160, 256, 5), (12288, 128, 6), (12304, 144, 4),
+                                       (13312, 256, 5)])
+def test_linear_many_k_groups(eng, oracle, inp, out, K):
+    """Inputs of 12, 13, 24, 25 and 26 k groups (512 elements each, the 13th and the 25th of one tile): the finisher folds
+    one row's partials in rounds of 12 groups and several rows' in rounds of 4, the staged path's finisher in rounds of
+    8 - the same left fold, so the same bits, and every row as it comes out alone."""
+    print(f"linear k groups {inp}x{out} K{K}", flush=True)
+    rng = np.random.default_rng(inp + out + K)
+    t, su, sv = synth.linear(rng, inp, out, K)
+    x = synth.bf16_values(rng, 9, inp)
+    lin = eng.exl3_linear(t, su, sv)
+    staged = eng.exl3_linear(t, su, sv).configure("staged", 1)
+    y = lin.run(x)
+    assert rel(y, oracle.exl3_linear(x, t, su, sv)) < 5e-5
+    assert np.array_equal(staged.run(x), y)
+    for R in (1, 2, 4):
+        assert np.array_equal(lin.run(x[:R]), y[:R]), R
+
+
 @pytest.mark.parametrize("R", [1, 4, 16])
 def test_linear_multi_launch_matches_single(eng, oracle, R):
     """q, k and v of config 3 (2048 -> 4096 / 512 / 512, K6) and a K5 linear recorded together
