@@ -58,10 +58,10 @@ struct ne_exl3_lin {
   uint32_t *tiles = nullptr;
   uint16_t *suh = nullptr, *svh = nullptr;
   uint16_t *xh = nullptr;  // [kLinMaxRows][in]
-  float *part = nullptr;   // [groups()][part_rows][OTp*16]: k group partials
+  float *part = nullptr;   // [S][R][OTp*16]: k group partials, room for part_floats
   uint32_t *cnt = nullptr; // per 128-column output block (the one-launch path's completion counters)
   bool one_launch = true;  // IJAH_LIN_PATH=staged at creation: prep, GEMM and finish as three launches
-  int part_rows = 0;
+  size_t part_floats = 0;
   float *hc_scr = nullptr;  // the HC read's scratch when this is its up linear (xn, u, ip), hc_rows rows
   int hc_rows = 0;
   ~ne_exl3_lin() {
@@ -209,20 +209,22 @@ struct LinScratch {
   float *part;
 };
 
-// LinArgs of one run at R rows (the k group partials grown to R rows as needed, or taken from sc)
+// LinArgs of one run at R rows (the k group partials grown as needed, or taken from sc)
 static LinArgs lin_args(ne_exl3_lin *l, int R, const float *x, float *y, const LinEpi &epi = LinEpi(),
                         const LinScratch *sc = nullptr) {
   const bool kloop = l->one_launch && l->k_loop(R);
   const bool wide = l->one_launch && epi.kind != 8 && l->k_wide(R);
   const int S = kloop ? 1 : l->groups();
-  if (!sc && R > l->part_rows) {  // never while the stream is captured: a captured launch would keep the freed buffer
+  const size_t need = (size_t)S * R * l->OTp * 16;  // (S differs by path: the row count alone would not tell)
+  if (!sc && need > l->part_floats) {  // never while the stream is captured: a captured launch would keep the freed buffer
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     IJ_HIP(hipStreamIsCapturing(stream(), &cs));
     IJ_CHECK(cs == hipStreamCaptureStatusNone, "linear: partial scratch must grow before a stream capture");
     dev_free(l->part);
-    // (room for every k group at any S: the paths that store fewer may be switched to one that stores them all)
-    l->part = dev_alloc<float>((size_t)l->groups() * R * l->OTp * 16);
-    l->part_rows = R;
+    l->part = nullptr;  // (the allocation may fail)
+    l->part_floats = 0;
+    l->part = dev_alloc<float>(need);
+    l->part_floats = need;
   }
   LinArgs a;
   a.tiles = l->tiles;
