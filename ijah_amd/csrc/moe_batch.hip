@@ -45,7 +45,6 @@ namespace {
 constexpr int kChunkRows = 128;   // rows of one GEMM chunk (4 matrix-core row blocks of 32)
 constexpr int64_t kRows32Below = 25, kRows64Below = 51;  // rows per expert that take 32- and 64-row chunks
 
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ void dma16(const void *src, void *lds_dst) {
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds_dst, 16, 0, 0);
 }
@@ -927,21 +926,20 @@ __device__ __forceinline__ void chunk_gemm(const uint16_t *A, int lda, int ahalf
   auto step = [&](auto nbc, int s, int sb) {
     constexpr int NB = decltype(nbc)::value;  // the chunk's row blocks: no branch inside the step
     TileWords w[4];
-    // (the steady count also serves the first DB steps, where more requests than that follow step s's data)
-    if (s + Io::DB < NS) {
-      __builtin_amdgcn_s_waitcnt(0x0F70 | kAfterSteady<Io::OA, Io::OB, DA>);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      read_step<K>(ring_b + sb * Io::PB, BL, w);
-      asm volatile("s_barrier" ::: "memory");
-      issue_a(s + DA, (sb + DA) % Io::RA);
-      issue_b(s + Io::DB, (sb + Io::DB) % Io::RB);
-    } else {
-      wait_vm15(after_step<Io::OA, Io::OB, DA, Io::DB>(s, NS));
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      read_step<K>(ring_b + sb * Io::PB, BL, w);
-      asm volatile("s_barrier" ::: "memory");
-      if (s + DA < NS) issue_a(s + DA, (sb + DA) % Io::RA);
-    }
+    ring_step<Io::OA, Io::OB, DA, Io::DB>(
+        s, NS,
+        [](auto n) {
+          if constexpr (std::is_same_v<decltype(n), int>)
+            wait_vm15(n);
+          else
+            __builtin_amdgcn_s_waitcnt(0x0F70 | decltype(n)::value);
+        },
+        [&](int) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous step's fragments are read
+          read_step<K>(ring_b + sb * Io::PB, BL, w);
+          asm volatile("s_barrier" ::: "memory");
+        },
+        [&](int j) { issue_a(j, (sb + DA) % Io::RA); }, [&](int j) { issue_b(j, (sb + Io::DB) % Io::RB); });
     const uint8_t *at = a_lane + (sb % Io::RA) * Io::AB;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -973,10 +971,7 @@ __device__ __forceinline__ void chunk_gemm(const uint16_t *A, int lda, int ahalf
       }
     }
   };
-  for (int j = 0; j < Io::DB && j < NS; j++) {
-    if (j < DA) issue_a(j, j % Io::RA);
-    issue_b(j, j);
-  }
+  ring_start<DA, Io::DB>(NS, [&](int j) { issue_a(j, j % Io::RA); }, [&](int j) { issue_b(j, j); });
   auto loop = [&](auto nbc) {
     for (int t0 = 0; t0 < NS; t0 += U) {
 #pragma unroll

@@ -7,6 +7,8 @@
 // Requests complete in issue order, so waiting until at most n are outstanding completes all but the last n.
 #pragma once
 
+#include <type_traits>
+
 namespace ijah {
 
 // How many requests were issued after A(t) and B(t), counted at step t before it issues: the s_waitcnt vmcnt that
@@ -44,8 +46,33 @@ static_assert(after_step<2, 1, 2, 5>(5, 1000) == kAfterSteady<2, 1, 2> &&
 // wait_vm15; a larger count waits as for 15, which only waits longer).
 template <int OA, int OB, int DA, int DB>
 constexpr int step_wait(int t, int NS) {
+  static_assert(kAfterSteady<OA, OB, DA> <= 15, "the wait's 4-bit count");
   const int n = after_step<OA, OB, DA, DB>(t, NS);
   return steady_step<DB>(t, NS) ? kAfterSteady<OA, OB, DA> : (n < 15 ? n : 15);
+}
+
+// The order itself, for the kernel and the host program alike. wait(n) makes all but the last n requests complete (n an
+// integral_constant in the steady state, so that the wait takes it as an immediate), ready(s) reads what the wave itself
+// requested for step s and passes the workgroup's barrier, a(j) and b(j) issue step j's requests.
+template <int DA, int DB, class A, class B>
+constexpr void ring_start(int NS, A a, B b) {
+  for (int j = 0; j < DB && j < NS; j++) {
+    if (j < DA) a(j);
+    b(j);
+  }
+}
+template <int OA, int OB, int DA, int DB, class W, class R, class A, class B>
+constexpr void ring_step(int s, int NS, W wait, R ready, A a, B b) {
+  if (steady_step<DB>(s, NS)) {
+    wait(std::integral_constant<int, kAfterSteady<OA, OB, DA>>{});
+    ready(s);
+    a(s + DA);
+    b(s + DB);
+  } else {
+    wait(step_wait<OA, OB, DA, DB>(s, NS));
+    ready(s);
+    if (s + DA < NS) a(s + DA);
+  }
 }
 
 }  // namespace ijah
