@@ -45,6 +45,15 @@ namespace {
 constexpr int kChunkRows = 128;   // rows of one GEMM chunk (4 matrix-core row blocks of 32)
 constexpr int64_t kRows32Below = 25, kRows64Below = 51;  // rows per expert that take 32- and 64-row chunks
 
+// The thread id as a value of its own from here on: what an epilogue derives from it is computed there and not held
+// through the k loop. With 64-row chunks (80 registers, so that three workgroups share a CU) the gate/up GEMM spilled 16 to
+// 18 registers, for such values and for scales held through the Hadamard, and reloaded two of them after its first
+// requests, which waited for all of those. Without any spills 1280, 1500, 2000 and 2400 rows at 2048 x 512, K5 take 475,
+// 500, 565 and 614 us a layer instead of 480, 509, 575 and 624.
+__device__ __forceinline__ int again(int tid) {
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
 __device__ __forceinline__ void dma16(const void *src, void *lds_dst) {
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds_dst, 16, 0, 0);
 }
@@ -1136,20 +1145,13 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
   //     chunk and stores them, 32 bytes.
   // (With H_4 as one of four outputs per lane, four multiply-adds per value on half the waves, and the H_4 of the last
   // step read whole rows from LDS again, the epilogues were 25% of the vector instructions here and 44% in bat_down.)
+  const int tid = again(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = wave & 3, n = lane & 31, h = lane >> 5;
   f16x8 hA1[2], hA2[2];
   h32_operand(lane, [](uint32_t m) { return m; }, hA1);
   h32_operand(lane, [](uint32_t m) { return kp_inv32(16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u)); }, hA2);
   const int e0 = 4 * wave + 2 * h;  // step 2's elements
   const float sc = a.sc_inter;
-  f16x2 sg[4], su[4], sd[4];  // their scales: columns 32 c + e0, + 1 of block ib
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    const int col = ib * 128 + 32 * c + e0;
-    sg[c] = *(const f16x2 *)((const uint16_t *)(blk + sv_of(a, e, 0)) + col);
-    su[c] = *(const f16x2 *)((const uint16_t *)(blk + sv_of(a, e, 1)) + col);
-    sd[c] = *(const f16x2 *)((const uint16_t *)(blk + su_of(a, e, 2)) + col);
-  }
   // LDS: 8 step-1 tiles of 32 rows x 32 elements, row pitch 36 floats; the 4 step-2 tiles take their place
   float *xt = (float *)lds;
   const int nrb = (nrows + 31) / 32;
@@ -1161,6 +1163,15 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_gateu
 #pragma unroll
     for (int g = 0; g < 4; g++)
       *(float4 *)(xt + (wave * 32 + n) * 36 + 8 * g + 4 * h) = make_float4(T[4 * g], T[4 * g + 1], T[4 * g + 2], T[4 * g + 3]);
+    // the scales of columns 32 c + e0, + 1 of block ib: per row block, so that they are not held through H_32
+    f16x2 sg[4], su[4], sd[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int col = ib * 128 + 32 * c + e0;
+      sg[c] = *(const f16x2 *)((const uint16_t *)(blk + sv_of(a, e, 0)) + col);
+      su[c] = *(const f16x2 *)((const uint16_t *)(blk + sv_of(a, e, 1)) + col);
+      sd[c] = *(const f16x2 *)((const uint16_t *)(blk + su_of(a, e, 2)) + col);
+    }
     __syncthreads();
     float hv[2][4];  // [element][chunk]
     {
@@ -1225,13 +1236,23 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
   int ch, ob2;
   if (!xcd_chunk((int)bk[3 * (a.ne + 1)], nob, ch, ob2)) return;
   const int e = (int)chunks[3 * ch], row0 = (int)chunks[3 * ch + 1], nrows = (int)chunks[3 * ch + 2];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = NR == 64 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)(threadIdx.x >> 6);
   const uint8_t *blk = expert_block(a, e);
-  // each row's slot (token, k) and route weight, gathered once into LDS (the slot ids requested before the GEMM)
+  // each row's slot (token, k) and route weight, gathered once into LDS (the slot ids requested before the GEMM; with 64-row
+  // chunks straight to LDS, as a register held through the k loop is one too many there, and ahead of the GEMM's own
+  // requests, so that its waits cover them)
   __shared__ uint32_t m_dst[kChunkRows];
   __shared__ float m_w[kChunkRows];
   const int mt = threadIdx.x;
-  const uint32_t sl = mt < nrows ? rows[row0 + mt] : 0u;
+  uint32_t sl = 0u;
+  if (mt < nrows) {
+    if constexpr (NR == 64)
+      __builtin_amdgcn_global_load_lds((const void *)(rows + row0 + mt),
+                                       (__attribute__((address_space(3))) void *)(m_dst + wave * 64), 4, 0, 0);
+    else
+      sl = rows[row0 + mt];
+  }
   constexpr int NRB = NR / 32;
   f32x16 acc[NRB];
   const uint16_t *A = hh + (uint64_t)row0 * a.inter;
@@ -1242,8 +1263,11 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
     chunk_gemm<K, 1, TR, NR, EX ? kFoldAll : 0>(A, a.inter, 0, 0, nrows, blk + tr_of(a, e, 2), a.inter / 16,
                                                 ob2 * 8 + wave, lds, acc, nullptr, 0, a.inter / 16);
   if (mt < nrows) {
+    if constexpr (NR == 64)
+      sl = m_dst[mt];
+    else
+      m_dst[mt] = sl;
     const int tok = sl / a.nslot, k = sl % a.nslot;
-    m_dst[mt] = sl;
     m_w[mt] = k >= a.topk ? a.sgv[tok] : __uint_as_float(a.route[(uint64_t)tok * 2 * a.topk + a.topk + k]);
   }
   if constexpr (!TR) {
@@ -1283,6 +1307,7 @@ __global__ __launch_bounds__(512, NR == kChunkRows || EX ? 4 : 6) void bat_down(
   // Per 32-row block: H_32 on the wave's tile (output element j = 16 h + i of the chunk at lane (n, h)), the tiles to
   // LDS; then wave w takes rows 4 w .. 4 w + 3 whole: lane (element j, block bb) reads its element of the block's four
   // chunks, and H_4 gives it the row's four columns 32 q + j, times 1/sqrt(128), svh_d and the slot's route weight.
+  const int tid = again(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   f16x8 hA[2];
   h32_operand(lane, [](uint32_t m) { return 16u * ((m >> 2) & 1u) + 4u * (m >> 3) + (m & 3u); }, hA);
   const int cb = lane >> 5, cj = lane & 31;

@@ -223,6 +223,19 @@ def test_moe_batch_chunk_sizes(eng, oracle, R, K, Ks):
     assert np.array_equal(same, np.repeat(y[:1], R, 0))
 
 
+@pytest.mark.parametrize("R,K,Ks", [(101, 5, 5), (203, 4, 4), (130, 6, 6), (166, 4, 5), (197, 6, 5), (100, 5, 6)])
+def test_moe_batch_64_row_chunks(eng, oracle, R, K, Ks):
+    """The form of 25 to 50 routed rows per expert (8 experts, top-2) at equal and at mixed widths: one and two row blocks
+    per chunk, remainders, and each row as it comes out in another order of the rows."""
+    print(f"moe batch 64-row chunks R{R} K{K}/{Ks}", flush=True)
+    w = synth.moe_layer(920 + R, hid=512, inter=256, ne=8, topk=2, K=K, shared=True, Ks=Ks, sgate=True)
+    W = oracle.MoeWeights(w)
+    m = eng.moe_create(w)
+    x = synth.bf16_values(np.random.default_rng(921), R, 512)
+    y, _ = check_layer(eng, oracle, m, W, x, exact=False)
+    assert np.array_equal(m.run(x[::-1])[::-1], y)
+
+
 def test_moe_batch_matches_staged(eng, oracle):
     """The grouped path and the staged kernels compute the same layer for several rows."""
     w = synth.moe_layer(81, hid=2048, inter=512, ne=64, topk=10, K=5, shared=True, Ks=5, sgate=False)

@@ -60,3 +60,11 @@ def test_linears_keep_four_waves(kernels, name):
     finisher, which one workgroup per output block runs, must not size the registers of all of them."""
     over = {n: k[".vgpr_count"] for n, k in _named(kernels, name).items() if k[".vgpr_count"] > 128}
     assert not over, over
+
+
+def test_no_kernel_spills_vector_registers(kernels):
+    """No kernel keeps vector registers in scratch memory: a reload waits for every earlier request of its wave, so in a
+    kernel that streams through LDS rings one spilled register drains the ring."""
+    over = {n: (k[".vgpr_spill_count"], k[".private_segment_fixed_size"]) for n, k in kernels.items()
+            if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
+    assert not over, over
