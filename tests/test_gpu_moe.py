@@ -574,6 +574,38 @@ def test_moe_fused_reference_shape(eng, oracle, shared, K, Ks):
         _rows_match_one_row(m, synth.bf16_values(np.random.default_rng(202), 4, 2560), 4)
 
 
+def _bf16_value(v):
+    return (synth.bf16(v.astype(np.float32)).astype(np.uint32) << 16).view(np.float32)
+
+
+def _low_part_rows(R, hid):
+    """rows whose odd 128-wide chunks are no bf16 values (their split has low parts); the first chunk only in the last row"""
+    rng = np.random.default_rng(R + hid)
+    x = rng.standard_normal((R, hid)).astype(np.float32)
+    for c in range(0, hid, 256):
+        x[:, c:c + 128] = _bf16_value(x[:, c:c + 128])
+    x[R - 1, :128] = rng.standard_normal(128)
+    return x
+
+
+@pytest.mark.parametrize("R,hid", [(33, 2048), (511, 512), (513, 512), (577, 1536)])
+def test_moe_router_low_parts(eng, R, hid):
+    """The matrix-core routers (up to 511 rows, and from 512) split f32 inputs into bf16 hi and lo, and the second leaves a
+    chunk's low products out where they are all zero. Logits against f64, rounded to bf16: the split is off by 2^-18 of each
+    input, so that fewer than 1 logit in 100 falls on the other side of a rounding boundary (0.2% do in a model of
+    the split); left out of a quarter of the inputs or more, or of the last row's first chunk, the low products (up to 2^-9 of
+    each input) move 17% or more of the logits that they belong to."""
+    print(f"moe router low parts R{R} hid{hid}", flush=True)
+    w = synth.moe_layer(930 + R, hid=hid, inter=128, ne=256, topk=2, K=4, shared=False, sgate=False)
+    m = eng.moe_create(w)
+    x = _low_part_rows(R, hid)
+    m.run(x)
+    router = (w["router"].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    off = m.read("logits", R) != _bf16_value(x.astype(np.float64) @ router.T)
+    assert off.mean() < 0.01
+    assert off[-1].mean() < 0.05  # one row: 256 logits, 1 or 2 of them expected
+
+
 def _rr(v):
     return synth.bf16(v.astype(np.float32)).astype(np.uint32).__lshift__(16).view(np.float32).astype(np.float64)
 
