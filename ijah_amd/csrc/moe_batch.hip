@@ -120,7 +120,7 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // A wave stages its own k range in LDS, 32 of k at a time (rows split on the way, whole 128-byte runs per load, kRsAhead
 // chunks' loads in flight): fragments loaded straight into registers, 16 scattered bytes a lane, kept the address units
-// busy for most of the 16.4 us that 48 rows took (now 13.3).
+// busy for most of the 16.4 us that 48 rows took (then 13.3; 11 under the kernel tracer).
 constexpr int kRouterWaves = 8;  // k splits
 constexpr int kRsKc = 32, kRsPitch = kRsKc + 8, kRsAhead = 4;
 constexpr int kRsWave = 3 * 32 * kRsPitch * 2;  // LDS bytes per wave: hi, lo, columns
@@ -814,16 +814,17 @@ __global__ __launch_bounds__(256) void bat_prep_rows(MoeArgs a, const uint32_t *
 }
 
 // ---------------------------------------------------------------------------------------------------- grouped GEMM
-// One workgroup (8 waves, two per SIMD) multiplies a chunk of up to NR expert-sorted rows of A by one tile pair (32
+// One workgroup (8 waves, two on each SIMD) multiplies a chunk of up to NR expert-sorted rows of A by one tile pair (32
 // columns) per wave of the expert's re-laid matrix (IT k tiles, IT even), two k tiles per step. There are NA A
 // operands (fp16, kp order, row stride lda halves, the second at A + ahalf): wave w multiplies operand aidx. Both
-// stream through LDS rings: A (shared; each wave requests 16 of its rows) kDA steps ahead, and each wave's own B
-// tiles kDB steps ahead, so that enough weight bytes are in flight per CU to cover the memory latency.
+// stream through LDS rings: A (shared; each wave requests NA NR / 8 of its rows) DA steps ahead, and each wave's own B
+// tiles DB steps ahead, so that enough weight bytes are in flight per CU to cover the memory latency.
 // acc[rb] = rows 32 rb.., the wave's 32 columns, in the matrix-core layout.
 constexpr int kWavesG = 8;
-// Two workgroups share a CU (so four waves per SIMD hide each other's latency): each keeps under 80 KB of LDS.
-// Steps (of 2 k tiles) requested ahead: A kDA, B kDB; the B ring's slot count is a multiple of the A ring's, so that
-// the k loop, unrolled by the B ring's length, addresses every ring slot with compile-time offsets.
+// At least two workgroups share a CU (so four waves per SIMD hide each other's latency): each keeps under 80 KB of LDS.
+// Steps (of 2 k tiles) requested ahead: A kDA, B kDB (64-row chunks: 1 and 3 at every K); the B ring's slot count is a
+// multiple of the A ring's, so that the k loop, unrolled by the B ring's length, addresses every ring slot with
+// compile-time offsets.
 template <int K>
 constexpr int kDA = K >= 6 ? 1 : 2;
 template <int K>
@@ -1635,7 +1636,7 @@ void launch_gemms_as(const MoeArgs &a, const MoeBatchBufs &b, hipStream_t s) {
   hipLaunchKernelGGL((bat_down<K, KS, TR, NR, EX>), dim3(g8 * (a.hid / 256)), dim3(64 * kWavesG),
                      ld, s, a, b.bk, b.chunks, b.rows, b.hh, b.dnw);
 }
-// Rows of a chunk (moe_gemm_rows) fix the form: 32-row chunks (eight waves per SIMD, row-major products and lane
+// Rows of a chunk (moe_gemm_rows) fix the form: 32-row chunks (at most 64 registers; row-major products and lane
 // butterflies, whose cost follows the rows) and, above, the transposed products and matrix-core Hadamard epilogues.
 // At most 32 rows (speculative verify) take the one-row step's arithmetic (every row bit-identical to the row run
 // alone).
@@ -1735,10 +1736,15 @@ bool moe_batch_supported(int K, int KS, int hid, int inter, int ne, int topk) {
   return ks && hid % 256 == 0 && inter % 128 == 0 && hid <= 8192 && inter <= 4096 && ne < 1024 && topk <= 32;
 }
 // Rows of a GEMM chunk by the routed rows per expert m. A chunk decodes its expert's weights once, whatever its rows,
-// so a chunk should hold an expert's rows whole; a smaller one runs with more workgroups per CU (4, 3 and 2) and
-// fetches fewer rows that are not there. Measured, hidden 2048 x inter 512, K5, us per layer at m = 4 / 14 / 20 / 25 /
-// 33 / 49: 32 rows 331 / 416 / 453 / 504 / 640 / 843, 64 rows 358 / 450 / 474 / 500 / 556 / 653, 128 rows 392 / 483 /
-// 505 / 530 / 586 / 677.
+// so a chunk should hold an expert's rows whole; a smaller one runs with more workgroups per CU (128 rows 2, 64 rows 3, by
+// registers; 32 rows 4, but gate/up at K5 3, by its rings' LDS) and fetches fewer rows that are not there. Measured, K5,
+// hidden 2048 x inter 512, us per layer (the least of three runs of eight), rows per expert across:
+//                4   14   20   24   28   33   44   49   52   55   64   80
+//    32 rows   320  403  438  480  526  617       832
+//    64 rows   354  433  451  472  497  529  610  632  661  700  819 1008
+//   128 rows   386  459  481  498  520  558  627  651  673  685  752  861
+// K4 (6-bit shared) and 2560 x 640 (8-bit shared) cross at the same m; K6 and 1024 x 256 cross to 128 rows at 56 to 58, where
+// the line at 51 costs them 1 to 4% between (K6 at m = 52: 687 and 715).
 static int moe_gemm_rows(int R, int ne, int topk) {
   const int64_t m = (int64_t)R * topk / ne;
   return m < kRows32Below ? 32 : m < kRows64Below ? 64 : kChunkRows;
