@@ -179,9 +179,9 @@ def test_moe_reference_shape_2560(eng, oracle, R):
 # ---------------------------------------------------------------------------------------------- batched path (R >= 2)
 @pytest.mark.parametrize("R", [16, 200, 640])
 def test_moe_batch_chunks(eng, oracle, R):
-    """R rows through the grouped matrix-core path: experts with more than one 128-row chunk (the shared expert at
-    R = 200, ~50 rows per routed expert), ties and order checked against the oracle on the GPU's route. R = 640 takes
-    the many-row router."""
+    """R rows through the grouped matrix-core path: experts with more than one chunk (at R = 200, 50 rows per routed expert
+    and 64-row chunks, the shared expert has four; at 640, 160 rows and 128-row chunks, routed ones have two), ties and order
+    checked against the oracle on the GPU's route. R = 640 takes the many-row router."""
     print(f"moe batch R{R}", flush=True)
     w = synth.moe_layer(70 + R, hid=1024, inter=256, ne=16, topk=4, K=5, shared=True, Ks=6, sgate=True)
     W = oracle.MoeWeights(w)
@@ -193,8 +193,8 @@ def test_moe_batch_chunks(eng, oracle, R):
 
 @pytest.mark.parametrize("R", [32, 33])
 def test_moe_batch_row_block_forms(eng, oracle, R):
-    """64 experts, top-10 + shared: at 32 rows the GEMMs take their one-row-block form and the shared expert fills a
-    whole 32-row chunk; at 33 rows the 128-row form (both row-major: few rows per routed expert)."""
+    """64 experts, top-10 + shared: 32 rows are the most that take the few-row kernels; 33 rows (5 per routed expert) take the
+    grouped GEMM with 32-row chunks, where the shared expert has one whole chunk and one of a single row."""
     print(f"moe batch forms R{R}", flush=True)
     w = synth.moe_layer(90 + R, hid=1024, inter=256, ne=64, topk=10, K=5, shared=True, Ks=5, sgate=True)
     W = oracle.MoeWeights(w)
