@@ -1745,6 +1745,10 @@ bool moe_batch_supported(int K, int KS, int hid, int inter, int ne, int topk) {
 //   128 rows   386  459  481  498  520  558  627  651  673  685  752  861
 // K4 (6-bit shared) and 2560 x 640 (8-bit shared) cross at the same m; K6 and 1024 x 256 cross to 128 rows at 56 to 58, where
 // the line at 51 costs them 1 to 4% between (K6 at m = 52: 687 and 715).
+// The launch is chosen on the host, which knows the mean alone. Uneven routing favours larger chunks: 1111 rows (m = 21) with
+// half of their variance in common take 455 / 408 / 412 us with 32- / 64- / 128-row chunks, and rows that all route alike
+// 338 / 266 / 236, the one kind of batch found that 128-row chunks at every size served better (274 us, with the decode and
+// epilogues of the time). Chunks of two sizes in one layer would take two more launches.
 static int moe_gemm_rows(int R, int ne, int topk) {
   const int64_t m = (int64_t)R * topk / ne;
   return m < kRows32Below ? 32 : m < kRows64Below ? 64 : kChunkRows;
